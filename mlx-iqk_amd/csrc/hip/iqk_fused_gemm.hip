@@ -23,7 +23,8 @@
 // there (dealing M-tile 8i + x to XCD x instead fetched 1.32x the unique
 // bytes from HBM, an expert's tiles landing on several XCDs).
 //
-// Tile: 512 threads, eight wavefronts.  Wavefront w owns weight rows
+// Tile (more than 16 slots; smaller ones take few_slots_tile): 512 threads,
+// eight wavefronts.  Wavefront w owns weight rows
 // 32w .. 32w+31 of the block (the 32 columns of v_mfma_f32_32x32x16_f16) for
 // all 64 slots (two 32-row MFMA blocks): two 16-register accumulators, so a
 // wavefront needs about 128 VGPRs and four fit per SIMD.
@@ -71,6 +72,7 @@ constexpr int kXChunks = 2 * kFusedKS / 16;      // 16-byte chunks of a staged r
 constexpr int kXRows = kFusedThreads / kXChunks; // rows one staging pass covers
 constexpr int kXPer = kFusedBM / kXRows;         // staging passes a step
 static_assert(kFusedBM % kXRows == 0 && kFusedThreads >= 256, "whole staging passes; the work-list scan needs 256 threads");
+constexpr uint32_t kNoStore = 0x7fffffffu;         // a slot without an output row: above any (n_slots <= 2^30)
 static_assert(kXRows == 32, "staging pass i is the 32-row MFMA slot block i");
 
 struct FusedArgs {
@@ -84,6 +86,50 @@ struct FusedArgs {
     uint32_t row_start;
     uint32_t n_groups, n_slots, n_x_rows;
 };
+
+struct FusedScan {
+    TileScan many;
+    uint32_t wave[kFusedWaves], group, mtile;
+};
+
+// The (group, M-tile) of an XCD's nth tile: XCD x takes tiles x ceil(T / 8) ..
+// of the list's T.  False (uniformly) past its share.  Up to a group a thread,
+// the sizes are loaded and scanned once, for T and the tile both.
+__device__ __forceinline__ bool claim_mtile(const uint32_t *offs, uint32_t n_groups, uint32_t xcd, uint32_t nth,
+                                            FusedScan &ts, uint32_t &group, uint32_t &mtile) {
+    if (n_groups > uint32_t(kFusedThreads)) {  // uniform
+        const uint32_t tiles = count_mtiles<kFusedBM, kFusedThreads>(offs, n_groups, ts.many);
+        const uint32_t per_xcd = (tiles + 7) / 8, tile = xcd * per_xcd + nth;
+        if (nth >= per_xcd || tile >= tiles) return false;
+        return find_mtile<kFusedBM, kFusedThreads>(offs, n_groups, tile, ts.many, group, mtile);
+    }
+    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const uint32_t cnt = tid < n_groups ? (offs[tid + 1] - offs[tid] + kFusedBM - 1) / kFusedBM : 0u;
+    uint32_t incl = cnt;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const uint32_t up = __shfl_up(incl, off, 64);
+        if (lane >= uint32_t(off)) incl += up;
+    }
+    if (lane == 63) ts.wave[wave] = incl;
+    __syncthreads();
+    uint32_t tiles = 0, before = 0;
+#pragma unroll
+    for (uint32_t w = 0; w < uint32_t(kFusedWaves); ++w) {
+        before += w < wave ? ts.wave[w] : 0u;
+        tiles += ts.wave[w];
+    }
+    const uint32_t per_xcd = (tiles + 7) / 8, tile = xcd * per_xcd + nth, excl = before + incl - cnt;
+    if (nth >= per_xcd || tile >= tiles) return false;  // uniform
+    if (tile - excl < cnt) {  // exactly one thread's
+        ts.group = tid;
+        ts.mtile = tile - excl;
+    }
+    __syncthreads();
+    group = ts.group;
+    mtile = ts.mtile;
+    return true;
+}
 
 // A block's scale planes in LDS.  IQ2_KS: scl u8 [K/64], sch u8 [K/256],
 // sex u8 [K/256], dv f16 per row.  IQ2_K: scl u16 [K/64], sex u8 [K/128],
@@ -239,6 +285,26 @@ __device__ __forceinline__ Pool scale_products(uint32_t n01, uint32_t n23, _Floa
     return {perm(p23, p01, 0x06040200u), perm(p23, p01, 0x07050301u)};
 }
 
+// IQ2_K's pools of the four 16-weight words of one u16 scale word scw
+// (nibble w: word w's index) and alphabet bits ab, under super-block scale dd.
+__device__ __forceinline__ void iq2k_pools(uint32_t scw, uint32_t ab, _Float16 dd, const uint2_t *ptab, Pool *p) {
+            // byte w: the table offset 8 (alpha_w << 4 | nibble_w) of word w; a
+            // v_perm spreads the scale word's bytes to (b0, b0, b1, b1), shifts
+            // put nibble w at bits 3-6 of byte w, and the multiply copies
+            // alphabet bit w to bit 8w (no two copies meet, so no carries;
+            // pinned, or it becomes a quarter-rate 32-bit multiply)
+            const uint32_t scp = perm(scw, scw, 0x01010000u);
+            uint32_t a8 = __umul24(ab, 0x204081u);
+            asm volatile("" : "+v"(a8));
+            const uint32_t kofs = ((scp << 3) & 0x00780078u) | ((scp >> 1) & 0x78007800u) | ((a8 & 0x01010101u) << 7);
+            const uint8_t *tab = reinterpret_cast<const uint8_t *>(ptab);
+#pragma unroll
+            for (int w = 0; w < 4; ++w) {
+                const uint2_t n = *reinterpret_cast<const uint2_t *>(tab + ((kofs >> (8 * w)) & 0xffu));
+                p[w] = scale_products(uint32_t(n.x), uint32_t(n.y), dd);
+            }
+}
+
 // The v_perm tables of lane (row, kg) at step s, one per 16-weight word of
 // its 64 weights: IQ2_KS sub-blocks 4s + 2kg + h (two words each), IQ2_K
 // sub-blocks 8s + 4kg + w (one word each).  IQ2_KS's tables are its exact
@@ -275,21 +341,7 @@ __device__ __forceinline__ void fused_pools(const FusedScales<MEMBER, K> &sc, in
             dd = half_of_bits(*reinterpret_cast<const uint16_t *>(sc.dv + row * S::DV_S + 2 * (s >> 1)));
         else
             dd = half_of_bits(dvw >> (16 * ((s >> 1) & 1)));
-        // byte w: the table offset 8 (alpha_w << 4 | nibble_w) of word w; a
-        // v_perm spreads the scale word's bytes to (b0, b0, b1, b1), shifts
-        // put nibble w at bits 3-6 of byte w, and the multiply copies
-        // alphabet bit w to bit 8w (no two copies meet, so no carries;
-        // pinned, or it becomes a quarter-rate 32-bit multiply)
-        const uint32_t scp = perm(scw, scw, 0x01010000u);
-        uint32_t a8 = __umul24(ab, 0x204081u);
-        asm volatile("" : "+v"(a8));
-        const uint32_t kofs = ((scp << 3) & 0x00780078u) | ((scp >> 1) & 0x78007800u) | ((a8 & 0x01010101u) << 7);
-        const uint8_t *tab = reinterpret_cast<const uint8_t *>(ptab);
-#pragma unroll
-        for (int w = 0; w < 4; ++w) {
-            const uint2_t n = *reinterpret_cast<const uint2_t *>(tab + ((kofs >> (8 * w)) & 0xffu));
-            p[w] = scale_products(uint32_t(n.x), uint32_t(n.y), dd);
-        }
+        iq2k_pools(scw, ab, dd, ptab, p);
     }
 }
 
@@ -346,6 +398,260 @@ __device__ __forceinline__ void expand_sel_paired(uint4_t sel, Pool p, uint32_t 
     }
 }
 
+// ---- tiles of few slots -----------------------------------------------------------
+
+constexpr int kFewSlots = 16;  // slots up to which a tile takes the path below
+
+__device__ __forceinline__ uint4_t buffer_u4(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) {
+    return __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0);
+}
+
+// A buffer of `bytes` from p: loads past it return zeros.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of(const void *p, uint64_t bytes) {
+    constexpr uint64_t kCap = 0xffffffffull;
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), 0, int(uint32_t(bytes < kCap ? bytes : kCap)),
+                                             0x00020000);
+}
+
+// The stream planes from stacked row row0 on, as buffers that end with the
+// stack: a lane addresses one by a 32-bit offset (no 64-bit address a lane
+// and plane, which the path below has no registers for), and a row past the
+// stack reads zeros.
+template <int MEMBER, int K>
+struct FewPlanes {
+    static constexpr int COUNT = MEMBER == IQ1_S_R4 ? 2 : 4;
+    static constexpr uint32_t ROW[4] = {MEMBER == IQ1_S_R4 ? K / 8 : K / 4,
+                                        MEMBER == IQ1_S_R4 ? K / 16 : MEMBER == IQ2_KS ? K / 64 : K / 32,
+                                        MEMBER == IQ2_KS ? K / 256 : K / 128, MEMBER == IQ2_KS ? K / 256 : K / 128};
+    __amdgpu_buffer_rsrc_t p[COUNT];
+
+    __device__ __forceinline__ FewPlanes(const FusedArgs &a, size_t row0) {
+        const size_t rows = size_t(a.n_groups) * a.out_rows - row0;
+        const void *s[4] = {a.s0, a.s1, a.s2, a.s3};
+#pragma unroll
+        for (int i = 0; i < COUNT; ++i) p[i] = buffer_of(static_cast<const uint8_t *>(s[i]) + row0 * ROW[i], rows * ROW[i]);
+    }
+};
+
+// One lane's weights of one row over a chunk of 512 reduction elements, in
+// the decode GEMV's layout: lane (n, g) = (l % 16, l / 16) of a 16-row block
+// holds row n; in step s (256 elements) of the chunk it takes 64 weights, the
+// IQ2 members' k = 256s + 64g .. +63, IQ1_S_R4's k = 128g + 64s .. +63, so the
+// four lanes of a row read 64 contiguous code bytes an instruction.
+template <int MEMBER, int K>
+struct FewLane {
+    uint4_t q[MEMBER == IQ1_S_R4 ? 1 : 2];  // code words (IQ1_S_R4: four blocks' index words)
+    uint32_t sc[2];                         // IQ2_KS: scl word a step; IQ2_K: scale u16 of both steps (sc[0]); IQ1_S_R4: qh words
+    uint32_t hb, ab;                        // IQ2_KS: sch, sex of both super-blocks; IQ2_K: dv pair, sex
+
+    // chunk c of row `row` (of the planes' first), lane group g
+    __device__ __forceinline__ void load(const FewPlanes<MEMBER, K> &pl, uint32_t row, int c, int g) {
+        using P = FewPlanes<MEMBER, K>;
+        if constexpr (MEMBER == IQ1_S_R4) {
+            q[0] = buffer_u4(pl.p[0], row * P::ROW[0] + 16 * g, 64 * c);
+            const uint2_t h = __builtin_amdgcn_raw_buffer_load_b64(pl.p[1], row * P::ROW[1] + 8 * g, 32 * c, 0);
+            sc[0] = h.x;
+            sc[1] = h.y;
+        } else {
+            q[0] = buffer_u4(pl.p[0], row * P::ROW[0] + 16 * g, 128 * c);
+            q[1] = buffer_u4(pl.p[0], row * P::ROW[0] + 64 + 16 * g, 128 * c);
+            if constexpr (MEMBER == IQ2_KS) {
+                const uint2_t v = __builtin_amdgcn_raw_buffer_load_b64(pl.p[1], row * P::ROW[1], 8 * c, 0);
+                sc[0] = v.x;
+                sc[1] = v.y;
+                hb = __builtin_amdgcn_raw_buffer_load_b16(pl.p[2], row * P::ROW[2], 2 * c, 0);
+                ab = __builtin_amdgcn_raw_buffer_load_b16(pl.p[3], row * P::ROW[3], 2 * c, 0);
+            } else {
+                sc[0] = __builtin_amdgcn_raw_buffer_load_b16(pl.p[1], row * P::ROW[1] + 2 * g, 16 * c, 0);
+                sc[1] = __builtin_amdgcn_raw_buffer_load_b16(pl.p[1], row * P::ROW[1] + 8 + 2 * g, 16 * c, 0);
+                ab = __builtin_amdgcn_raw_buffer_load_b32(pl.p[2], row * P::ROW[2], 4 * c, 0);
+                hb = __builtin_amdgcn_raw_buffer_load_b32(pl.p[3], row * P::ROW[3], 4 * c, 0);
+            }
+        }
+    }
+
+    // The v_perm tables of step s's four 16-weight words, and (IQ1_S_R4) the
+    // words' pool selectors.
+    __device__ __forceinline__ void tables(int s, int g, const uint2_t *ptab, const uint2_t *grid, Pool *p,
+                                           uint4_t *sels) const {
+        if constexpr (MEMBER == IQ1_S_R4) {
+            fused_iq1(uint4_t{s ? q[0].z : q[0].x, s ? q[0].w : q[0].y, sc[s], 0u}, grid, ptab, p, sels);
+        } else if constexpr (MEMBER == IQ2_KS) {
+            const uint32_t scl = sc[s] >> (8 * g);  // nibbles of sub-blocks 2g, 2g+1
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const int bit = 8 * s + 2 * g + h;
+                const uint32_t e = ((scl >> (4 * h)) & 15u) | (((hb >> bit) & 1u) << 4) | (((ab >> bit) & 1u) << 5);
+                const uint2_t v = ptab[e];
+                p[2 * h] = {v.x, v.y};
+                p[2 * h + 1] = p[2 * h];
+            }
+        } else {
+            iq2k_pools(sc[s], (ab >> (16 * s + 4 * g)) & 15u, half_of_bits((hb >> (16 * s)) & 0xffffu), ptab, p);
+        }
+    }
+
+    __device__ __forceinline__ uint32_t word(int s, int w) const { return q[MEMBER == IQ1_S_R4 ? 0 : s][w]; }
+};
+
+// A tile of at most ROWS (8 or 16) slots against the block's 256 weight rows,
+// on v_mfma_f32_16x16x32_f16.  Most experts of a batch or a short prompt have
+// such tiles only, and the work is then one expansion of every routed weight
+// beside one read of its streams.  The 32-slot MFMAs of the larger tiles ran
+// half empty or worse there, and a barrier every 128 elements held all eight
+// wavefronts to the slowest one's loads.  Here a wavefront (32 rows, two
+// 16-row blocks sharing every A read) keeps a chunk of 512 elements in flight
+// while it expands another, and the activations are staged by phases of PC
+// chunks, as many as 64 KB hold (IQ1_S_R4, beside its grid: 32 KB): between
+// two phases the wavefronts run free of one another.
+//
+// What bounds it: VALU issue.  Taking the loads out leaves 88% of the time,
+// the MFMAs 86%, and 16-row wavefronts at six or eight a SIMD measured the
+// same, as did loads of whole rows turned through LDS.  The line at 16 slots:
+// two 16-slot blocks an operand measured 5% slower than one 32-slot MFMA
+// (1024 tokens, uniform: 24 slots an expert).  Measured (the kernel alone, 256
+// experts, top-6, uniform routing, IQ2_KS gate): 24 tokens 102 -> 84 us, 64
+// 176 -> 144, 128 209 -> 171, 512 227 -> 207; Zipf(1.1) routing: IQ2_KS gate
+// 64 tokens 112 -> 94, 512 243 -> 227, IQ1_S_R4 gate 143 -> 123 and 235 -> 205
+// (128 and 512), IQ2_K down 166 -> 157 and 271 -> 254; 2048 tokens 386 -> 369,
+// 377 -> 356, 430 -> 418.
+template <int MEMBER, int K, int ROWS, int PC>
+struct FewShape {
+    static constexpr int PHASE = 512 * PC;           // reduction elements staged at once
+    static constexpr int STRIDE = 2 * PHASE + 16;    // LDS bytes per staged row
+    static constexpr int BYTES = ROWS * STRIDE;
+    static constexpr int UNITS = 2 * PHASE / 16;     // 16-byte units a row
+};
+
+template <int MEMBER, int K, int ROWS, int PC>
+__device__ __forceinline__ void few_slots_tile(const FusedArgs &a, uint8_t *xs, uint32_t *slot_dst, uint32_t *slot_x,
+                                               const uint2_t *ptab, const uint2_t *grid, uint32_t m0, uint32_t gend,
+                                               uint32_t n0, int rows_here, size_t row0, int tid) {
+    constexpr bool IQ1 = MEMBER == IQ1_S_R4;
+    using F = FewShape<MEMBER, K, ROWS, PC>;
+    constexpr int CHUNKS = K / 512;
+    static_assert(CHUNKS % 2 == 0 && CHUNKS % PC == 0, "chunks go in pairs, whole phases");
+    const int wave = tid >> 6, l = tid & 63, n = l & 15, g = l >> 4;
+    // rows 32 wave + 16 r + n; one past the range reads what follows it (zeros
+    // past the stack) and is not stored
+    using Lane = FewLane<MEMBER, K>;
+    const FewPlanes<MEMBER, K> planes(a, row0);
+    const uint32_t wrow = uint32_t(32 * wave + n);
+    Lane cur[2], nxt[2];
+#pragma unroll
+    for (int r = 0; r < 2; ++r) cur[r].load(planes, wrow + 16 * r, 0, g);
+    // each slot's activation row (bytes into x; past x's buffer, so zeros, if
+    // it has none) and output row
+    const uint32_t xbytes = a.n_x_rows * uint32_t(2 * K);  // below 4 GiB (the entry point)
+    const __amdgpu_buffer_rsrc_t xbuf = buffer_of(a.x, xbytes);
+    if (tid < kFewSlots) {
+        const uint32_t xp = m0 + uint32_t(tid);
+        uint32_t off = xbytes, dst = kNoStore;
+        if (xp < gend) {
+            const uint32_t row = a.xr[xp], yrow = a.yr ? a.yr[xp] : xp;
+            if (row < a.n_x_rows) off = row * uint32_t(2 * K);
+            if (yrow < a.n_slots) dst = yrow | (row < a.n_x_rows ? 0x80000000u : 0u);  // else NaN
+        }
+        slot_dst[tid] = dst;
+        slot_x[tid] = off;
+    }
+    const int live = int(min(gend - m0, uint32_t(ROWS)));
+    // phase ph: units (16 bytes, in the paired order of expand_word_paired) of
+    // the live rows, four loads in flight a thread.  IQ1_S_R4's chunks are
+    // stored as the lanes take them: [step][lane group][64 elements].
+    const auto stage = [&](int ph) {
+        const int units = live * F::UNITS;
+        for (int u0 = 0; u0 < units; u0 += 4 * kFusedThreads) {
+            uint4_t v[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int u = u0 + kFusedThreads * i + tid, row = u / F::UNITS, c = u % F::UNITS;
+                if (row < live) v[i] = buffer_u4(xbuf, slot_x[row] + 16 * c, 2 * F::PHASE * ph);
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int u = u0 + kFusedThreads * i + tid, row = u / F::UNITS;
+                int c = u % F::UNITS;
+                if constexpr (IQ1) c = (c & ~63) | ((c & 8) << 2) | ((c & 48) >> 1) | (c & 7);
+                if (row < live)
+                    *reinterpret_cast<uint4_t *>(xs + row * F::STRIDE + 16 * c) =
+                        uint4_t{perm(v[i].z, v[i].x, 0x05040100u), perm(v[i].z, v[i].x, 0x07060302u),
+                                perm(v[i].w, v[i].y, 0x05040100u), perm(v[i].w, v[i].y, 0x07060302u)};
+            }
+        }
+    };
+    __syncthreads();  // the slots' rows, the tables
+    stage(0);
+    __syncthreads();
+
+    float4_t acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+    // a lane whose slot is past the tile's last reads one of its live rows:
+    // its products reach only its own output row, never stored
+    const uint8_t *abase = xs + min(n, max(live - 1, 0)) * F::STRIDE + 128 * g;
+    const auto chunk = [&](int c, const Lane (&now)[2], Lane (&then)[2]) {
+        if (c > 0 && c % PC == 0) {
+            __syncthreads();  // every wavefront is done with the last phase
+            stage(c / PC);
+            __syncthreads();
+        }
+        if (c + 1 < CHUNKS) {
+#pragma unroll
+            for (int r = 0; r < 2; ++r) then[r].load(planes, wrow + 16 * r, c + 1, g);
+        }
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+            Pool p[2][4];
+            uint4_t sels[2][IQ1 ? 4 : 1];
+#pragma unroll
+            for (int r = 0; r < 2; ++r) now[r].tables(s, g, ptab, grid, p[r], sels[r]);
+            const int aoff = 1024 * (c % PC) + 512 * s;
+#pragma unroll
+            for (int w = 0; w < 4; ++w) {
+                half8_t af[2];
+#pragma unroll
+                for (int h = 0; h < 2; ++h)
+                    af[h] = __builtin_bit_cast(half8_t, *reinterpret_cast<const uint4_t *>(abase + aoff + 32 * w + 16 * h));
+#pragma unroll
+                for (int r = 0; r < 2; ++r) {
+                    uint32_t bw[8];
+                    if constexpr (IQ1)
+                        expand_sel_paired(sels[r][w], p[r][w], bw);
+                    else
+                        expand_word_paired(now[r].word(s, w), p[r][w], bw);
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) {
+                        const half8_t bf =
+                            __builtin_bit_cast(half8_t, uint4_t{bw[h], bw[2 + h], bw[4 + h], bw[6 + h]});
+                        acc[r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[h], bf, acc[r], 0, 0, 0);
+                    }
+                }
+            }
+        }
+    };
+#pragma unroll 1
+    for (int c = 0; c < CHUNKS; c += 2) {
+        chunk(c, cur, nxt);
+        chunk(c + 1, nxt, cur);
+    }
+
+    // D (16x16): lane (n, g), register i holds slot 4g + i of weight row n
+#pragma unroll
+    for (int r = 0; r < 2; ++r) {
+        const int lrow = 32 * wave + 16 * r + n;
+        if (lrow >= rows_here) continue;
+        float d = 1.f;  // the row scale of the sums; IQ2_K's scales are in its pools
+        if constexpr (MEMBER == IQ2_KS) d = float(half_of_bits(static_cast<const uint16_t *>(a.s4)[row0 + lrow]));
+        if constexpr (IQ1) d = float(half_of_bits(static_cast<const uint16_t *>(a.s2)[row0 + lrow]));
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const uint32_t dst = slot_dst[4 * g + i];
+            if (dst != kNoStore)
+                a.y[size_t(dst & 0x7fffffffu) * a.N + n0 + lrow] =
+                    (dst >> 31) ? uint16_t(float_to_half_bits(MEMBER == IQ2_K ? acc[r][i] : acc[r][i] * d)) : kHalfNaN;
+        }
+    }
+}
+
 template <int MEMBER, int K>
 __global__ __launch_bounds__(kFusedThreads) __attribute__((amdgpu_waves_per_eu(4)))
 void fused_gemm_kernel(FusedArgs a) {
@@ -359,26 +665,35 @@ void fused_gemm_kernel(FusedArgs a) {
     // group, a line of their code plane is loaded four times, not 8 or 16.
     constexpr int G = IQ1 ? 4 : 1;
     static_assert(STEPS % G == 0, "whole groups of steps");
-    __shared__ TileScan ts;
-    __shared__ __attribute__((aligned(16))) uint8_t xs[2][kFusedBM * kXStride];
+    __shared__ FusedScan ts;
     // per slot of the tile: its output row, bit 31 set when its activations
     // are real (else its output row is NaN), or kNoStore
     __shared__ uint32_t slot_dst[kFusedBM];
+    __shared__ uint32_t slot_x[kFewSlots];
     __shared__ uint2_t ptab[MEMBER == IQ2_K ? 32 : IQ1 ? 16 : 64];  // pool products (IQ2_K) or pools
-    constexpr uint32_t kNoStore = 0x7fffffffu;  // above any row (n_slots <= 2^30)
-    __shared__ __attribute__((aligned(16))) std::conditional_t<IQ1, FusedGrid, S> sc;
+    // Phases of a few-slot tile: 64 KB of activations beside the tables leave
+    // two blocks a CU; IQ1_S_R4's grid leaves room for 32 KB.
+    constexpr int P8 = IQ1 ? 4 : 8, PC8 = P8 < K / 512 ? P8 : K / 512;
+    using F8 = FewShape<MEMBER, K, 8, PC8>;
+    using F16 = FewShape<MEMBER, K, 16, P8 / 2>;
+    constexpr int GRID_BYTES = IQ1 ? int(sizeof(FusedGrid)) : 0;
+    constexpr int XS_BYTES = 2 * kFusedBM * kXStride;
+    constexpr int WIDE_BYTES = XS_BYTES + (IQ1 ? 0 : int(sizeof(S)));
+    constexpr int FEW_BYTES = F16::BYTES;
+    static_assert(F8::BYTES <= FEW_BYTES && XS_BYTES % 16 == 0, "LDS sized for every form");
+    __shared__ __attribute__((aligned(16))) uint8_t smem[GRID_BYTES + (WIDE_BYTES > FEW_BYTES ? WIDE_BYTES : FEW_BYTES)];
+    uint2_t *const grid = reinterpret_cast<uint2_t *>(smem);  // IQ1_S_R4
+    uint8_t *const fxs = smem + GRID_BYTES;
+    auto &xs = *reinterpret_cast<uint8_t (*)[2][kFusedBM * kXStride]>(fxs);
+    S &sc = *reinterpret_cast<S *>(fxs + (IQ1 ? 0 : XS_BYTES));
 
     const int tid = threadIdx.x;
     const uint32_t ncb = (a.N + kFusedBN - 1) / kFusedBN;  // column blocks
-    const uint32_t tiles = count_mtiles<kFusedBM, kFusedThreads>(a.offs, a.n_groups, ts);
-    const uint32_t per_xcd = (tiles + 7) / 8;
-    const uint32_t xcd = blockIdx.x & 7u, j = blockIdx.x >> 3;
-    if (j / ncb >= per_xcd) return;  // surplus block (uniform)
-    const uint32_t tile = xcd * per_xcd + j / ncb, cblock = j % ncb;
-    if (tile >= tiles) return;
+    const uint32_t xcd = blockIdx.x & 7u, j = blockIdx.x >> 3, cblock = j % ncb;
     uint32_t g, mtile;
-    if (!find_mtile<kFusedBM, kFusedThreads>(a.offs, a.n_groups, tile, ts, g, mtile)) return;
+    if (!claim_mtile(a.offs, a.n_groups, xcd, j / ncb, ts, g, mtile)) return;  // surplus block (uniform)
     g = __builtin_amdgcn_readfirstlane(g);  // uniform (read from LDS): the stream bases stay scalar
+    mtile = __builtin_amdgcn_readfirstlane(mtile);
 
     // Offsets and row indices are device data: a slot outside [0, n_slots)
     // is never stored, a row outside x is never read (its output row is NaN),
@@ -399,16 +714,28 @@ void fused_gemm_kernel(FusedArgs a) {
     } else {
         if (tid < 64) ptab[tid] = kIq2ksPools.p[tid];
     }
-    // scale planes of the block's rows (IQ1_S_R4: the grid as pool selectors)
-    if constexpr (IQ1) {
+    if constexpr (IQ1) {  // the grid as pool selectors
         static_assert(IQK_IQ1S_GRID_SIZE == 4 * kFusedThreads, "four grid entries a thread");
         const uint2_t cw = reinterpret_cast<const uint2_t *>(iqk_iq1s_grid_codes)[tid];
 #pragma unroll
         for (int i = 0; i < 4; ++i)
-            sc.sel[4 * tid + i] = grid_selectors(((i < 2 ? cw.x : cw.y) >> (16 * (i & 1))) & 0xffffu);
-    } else {
-        copy_plane<S::SCL, S::SCL_S>(static_cast<const uint8_t *>(a.s1) + row0 * S::SCL, rows_here, sc.scl, tid);
+            grid[4 * tid + i] = grid_selectors(((i < 2 ? cw.x : cw.y) >> (16 * (i & 1))) & 0xffffu);
     }
+    // Few slots (uniform per block).  The empty asm keeps the forms' code
+    // apart: merged ahead of the branches it costs each of them registers.
+    if (gend - m0 <= 8u) {
+        asm volatile("" ::"n"(8));
+        few_slots_tile<MEMBER, K, 8, PC8>(a, fxs, slot_dst, slot_x, ptab, grid, m0, gend, n0, rows_here, row0, tid);
+        return;
+    }
+    if (gend - m0 <= uint32_t(kFewSlots)) {
+        asm volatile("" ::"n"(16));
+        few_slots_tile<MEMBER, K, 16, P8 / 2>(a, fxs, slot_dst, slot_x, ptab, grid, m0, gend, n0, rows_here, row0, tid);
+        return;
+    }
+    // scale planes of the block's rows
+    if constexpr (!IQ1)
+        copy_plane<S::SCL, S::SCL_S>(static_cast<const uint8_t *>(a.s1) + row0 * S::SCL, rows_here, sc.scl, tid);
     if constexpr (MEMBER == IQ2_KS) {
         copy_plane<S::HB, S::HB_S>(static_cast<const uint8_t *>(a.s2) + row0 * S::HB, rows_here, sc.hb, tid);
         copy_plane<S::EX, S::EX_S>(static_cast<const uint8_t *>(a.s3) + row0 * S::EX, rows_here, sc.ex, tid);
@@ -562,10 +889,9 @@ void fused_gemm_kernel(FusedArgs a) {
     else if constexpr (IQ1)
         d = half_of_bits(static_cast<const uint16_t *>(a.s2)[row0 + wl]);
 
-    // A tile of at most 32 real slots (most experts of a skewed routing)
-    // runs the second slot block's MFMAs for nothing: skip them (its slots
-    // 32 .. 63 are past the tile's end, never stored, so their accumulators
-    // do not exist).
+    // A tile of at most 32 real slots runs the second slot block's MFMAs for
+    // nothing: skip them (its slots 32 .. 63 are past the tile's end, never
+    // stored, so their accumulators do not exist).
     const auto run_steps = [&](auto slot_blocks) {
         constexpr int MB = decltype(slot_blocks)::value;
         float16_t acc[MB];
@@ -587,7 +913,7 @@ void fused_gemm_kernel(FusedArgs a) {
             uint32_t words[4];
             uint4_t sels[IQ1 ? 4 : 1];
             if constexpr (IQ1) {
-                fused_iq1(group_step(grp, j), sc.sel, ptab, p, sels);
+                fused_iq1(group_step(grp, j), grid, ptab, p, sels);
             } else {
                 // the lane's sub-blocks are those the one-step order gives
                 // step G(s/G) + kg's lane group j

@@ -1,0 +1,90 @@
+"""The fused prefill GEMM at the edges of its tile forms.
+
+A tile holds up to 64 slots of one expert; tiles of at most 8, at most 16, at
+most 32 and more slots run different code, and the work list is scanned in one
+pass for up to 512 experts.  One call here has experts of every count around
+those edges, over whole and partial blocks of 256 weight rows, with a slot
+without an activation row; every output is compared with a float64
+contraction of the oracle's weights.
+
+Tolerance: the operands are fp16 and the sums f32, so an output differs from
+float64 by its own fp16 rounding (2^-11), for IQ2_K by the weights' too (2^-11
+a term, about 2^-11 of the result), and by f32 sums of 4096 terms (under
+2^-13): 2e-3 of the largest output is above twice their sum.
+"""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+import wirepack
+from mlx_iqk_amd import format as fmt
+from mlx_iqk_amd import kernels
+from mlx_iqk_amd.nn import IqkSwitchLinear
+from oracle import oracle
+
+pytestmark = pytest.mark.gpu
+
+
+def _module(member, experts, out, n, seed, device):
+    wire = wirepack.random_wire(member, experts * out, n, seed=seed, scales="serving")
+    module = IqkSwitchLinear(member, experts, out, n, device=device)
+    module.load_wire(torch.from_numpy(wire).to(device))
+    return module, oracle.dequantize(member, wire, n).reshape(experts, out, n)
+
+
+def _call(module, counts, device, seed, row_start, rows, dead):
+    """Slots sorted by expert, each with an activation row of its own choosing;
+    slot `dead` names a row past x.  Returns y, x and the slots' rows."""
+    rng = np.random.default_rng(seed)
+    P, n = int(np.sum(counts)), module.in_features
+    n_x = max(1, P // 2)
+    x = rng.standard_normal((n_x, n)).astype(np.float16)
+    xr = rng.integers(0, n_x, P).astype(np.int32)
+    xr[dead] = n_x + 3
+    yr = rng.permutation(P).astype(np.int32)
+    offs = np.concatenate([[0], np.cumsum(counts)]).astype(np.int32)
+    y = kernels.fused_matmul(module.member, torch.from_numpy(x).to(device), module._streams(), module.num_experts,
+                             module.out_features, *(torch.from_numpy(a).to(device) for a in (offs, xr, yr)),
+                             row_start=row_start, rows=rows)
+    return y[torch.from_numpy(yr.astype(np.int64)).to(device)].float().cpu().numpy(), x, xr
+
+
+def _check(got, x, xr, counts, weights, dead):
+    e_of = np.repeat(np.arange(len(counts)), counts)
+    assert np.isnan(got[dead]).all()
+    live = np.arange(len(xr)) != dead
+    assert np.isfinite(got[live]).all()
+    want = np.empty(got.shape)
+    for e in np.unique(e_of):
+        s = np.nonzero((e_of == e) & live)[0]
+        want[s] = x[xr[s]].astype(np.float64) @ weights[e].astype(np.float64).T
+    assert np.max(np.abs(got[live] - want[live])) <= 2e-3 * np.max(np.abs(want[live]))
+
+
+COUNTS = [1, 0, 7, 8, 9, 15, 16, 17, 31, 32, 33, 63, 64, 65, 72, 73, 80, 81, 96, 97, 128, 129, 2]
+
+
+@pytest.mark.parametrize("member", fmt.MEMBERS)
+@pytest.mark.parametrize("n", kernels.SUPPORTED_IN_FEATURES)
+@pytest.mark.parametrize("out,row_start,rows", [(272, 0, 272), (272, 13, 259), (16, 0, 16)])
+def test_every_tile_form_matches_float64(device, member, n, out, row_start, rows):
+    print(f"fused tiles {member} n={n} out={out} rows [{row_start}, +{rows})", flush=True)
+    seed = wirepack.seed_for(member, n, out, "tiles")
+    module, ref = _module(member, len(COUNTS), out, n, seed, device)
+    dead = int(np.sum(COUNTS[:4])) + 2  # within the expert of nine slots
+    got, x, xr = _call(module, COUNTS, device, seed, row_start, rows, dead)
+    _check(got, x, xr, COUNTS, ref[:, row_start:row_start + rows], dead)
+
+
+@pytest.mark.parametrize("experts", (511, 512, 513, 600))
+def test_more_experts_than_one_scan(device, experts):
+    print(f"fused tiles over {experts} experts", flush=True)
+    rng = np.random.default_rng(experts)
+    counts = rng.choice([0, 1, 2, 9, 20, 70], size=experts, p=[0.5, 0.3, 0.1, 0.05, 0.03, 0.02])
+    counts[[0, -1]] = [5, 66]
+    module, ref = _module("iq2_ks", experts, 16, 2048, 7, device)
+    got, x, xr = _call(module, counts, device, 11, 0, 16, dead=3)
+    _check(got, x, xr, counts, ref, dead=3)
