@@ -36,7 +36,7 @@
 extern "C" {
 #endif
 
-#define IQK_HIP_ABI_VERSION 5
+#define IQK_HIP_ABI_VERSION 6
 
 #define IQK_MEMBER_IQ2_KS 0
 #define IQK_MEMBER_IQ2_K 1
@@ -69,6 +69,14 @@ int iqk_gemv(int member, int64_t in_features, int64_t out_features, int64_t num_
              const void *x, const void *const *streams, int n_streams,
              const uint32_t *sel, uint32_t pairs_per_row, uint32_t mats,
              void *y, void *stream);
+
+// The same with 64-bit expert ids (sel: i64 [mats], as torch.topk gives them);
+// one outside [0, num_experts) gives a NaN row.  A dispatch reads its ids
+// itself, so a caller's int64 ids cost no conversion launches.
+int iqk_gemv_ids64(int member, int64_t in_features, int64_t out_features, int64_t num_experts,
+                   const void *x, const void *const *streams, int n_streams,
+                   const int64_t *sel, uint32_t pairs_per_row, uint32_t mats,
+                   void *y, void *stream);
 
 // The GEMV's deleted-decode floor: identical loads, the decode replaced by an
 // integer fold of every loaded word that reaches y (reference:
@@ -219,6 +227,11 @@ int iqk_fused_gemm(int member, int64_t in_features, int64_t out_features, int64_
 int iqk_route(const uint32_t *ids, int64_t n_pairs, int64_t num_experts, int64_t rows_per_pair,
               int64_t pairs_per_x_row, int64_t n_x_rows, uint32_t *group_offsets, uint32_t *x_rows,
               uint32_t *y_rows, void *stream);
+
+// The same with 64-bit expert ids (ids: i64 [n_pairs]).
+int iqk_route_ids64(const int64_t *ids, int64_t n_pairs, int64_t num_experts, int64_t rows_per_pair,
+                    int64_t pairs_per_x_row, int64_t n_x_rows, uint32_t *group_offsets, uint32_t *x_rows,
+                    uint32_t *y_rows, void *stream);
 
 // ik wire rows -> the member's relayout streams, on the GPU (replaces
 // format.pack for rows already in device memory, src/mlx_iqk/format.py:478-588,

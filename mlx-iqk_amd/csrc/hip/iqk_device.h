@@ -60,6 +60,15 @@ struct TransposeReduce {
     }
 };
 
+// Expert id of pair m: ids holds 32-bit ids (wide = 0) or 64-bit ones (wide =
+// 1: little-endian word pairs), of which one outside [0, 2^32) reads as
+// 0xffffffff, an id no stack has.
+__device__ __forceinline__ uint32_t expert_id(const uint32_t *ids, uint32_t m, uint32_t wide) {
+    const size_t i = size_t(m) << wide;
+    const uint32_t high = ids[i | wide] & (0u - wide);
+    return high ? 0xffffffffu : ids[i];
+}
+
 __device__ __forceinline__ int lane_id() { return int(__lane_id()); }
 
 // Shared memory of the grouped work-list scan.

@@ -41,6 +41,7 @@ struct GemvArgs {
     uint32_t pairs_per_row;
     uint32_t num_experts;
     uint32_t out_features;
+    uint32_t wide_ids;  // 1: sel holds 64-bit ids
     uint16_t *y;
 };
 
@@ -136,7 +137,7 @@ __global__ __launch_bounds__(64) void gemv_kernel(GemvArgs a) {
     const int lc = lane % LPR, rsub = lane / LPR;
     const uint32_t m = blockIdx.y;
     const uint32_t row0 = blockIdx.x * 16;
-    const uint32_t e = a.sel[m];
+    const uint32_t e = expert_id(a.sel, m, a.wide_ids);
     const uint32_t tok = a.toks ? a.toks[m] : m / a.pairs_per_row;
     uint16_t *yrow = a.y + size_t(m) * a.out_features + row0;
     if (e >= a.num_experts || tok >= a.n_x_rows) {
@@ -299,8 +300,8 @@ int launch_gemv(int64_t n, const GemvArgs &a, uint32_t mats, hipStream_t st) {
 // The int8-MFMA path (iqk_gemv_mfma.hip); -1 when it does not apply.
 int gemv_mfma_dispatch(int floor, int member, int64_t n, int64_t out, int64_t num_experts, const void *x,
                        int64_t n_x_rows, const void *const *streams, int n_streams, const uint32_t *sel,
-                       const uint32_t *toks, bool union_runs, uint32_t pairs_per_row, uint32_t mats, void *y,
-                       hipStream_t st);
+                       bool wide_ids, const uint32_t *toks, bool union_runs, uint32_t pairs_per_row, uint32_t mats,
+                       void *y, hipStream_t st);
 
 // All GEMV entry points.  toks NULL: pair m reads x row m / pairs_per_row
 // (n_x_rows = mats / pairs_per_row); else x row toks[m] < n_x_rows (a row
@@ -311,7 +312,8 @@ int gemv_mfma_dispatch(int floor, int member, int64_t n, int64_t out, int64_t nu
 template <int FLOOR>
 int gemv_entry(int member, int64_t n, int64_t out, int64_t num_experts, const void *x, int64_t n_x_rows,
                const void *const *streams, int n_streams, const uint32_t *sel, const uint32_t *toks,
-               uint32_t pairs_per_row, uint32_t mats, void *y, void *stream, bool union_runs = false) {
+               uint32_t pairs_per_row, uint32_t mats, void *y, void *stream, bool union_runs = false,
+               bool wide_ids = false) {
     const int g = iqk_check_gemv_geometry(member, n, out);
     if (g != IQK_OK) return g;
     if (toks && member == IQK_MEMBER_IQ1_S_R4) return IQK_ERR_MEMBER;  // no sorted/union form
@@ -325,7 +327,7 @@ int gemv_entry(int member, int64_t n, int64_t out, int64_t num_experts, const vo
     if (mats > 65535u) return IQK_ERR_ARGUMENT;
     hipStream_t st = as_stream(stream);
     const int r = gemv_mfma_dispatch(FLOOR, member, n, out, num_experts, x, n_x_rows, streams, n_streams, sel,
-                                     toks, union_runs, pairs_per_row, mats, y, st);
+                                     wide_ids, toks, union_runs, pairs_per_row, mats, y, st);
     if (r >= 0) return r;
     GemvArgs a;
     a.x = static_cast<const uint32_t *>(x);
@@ -338,6 +340,7 @@ int gemv_entry(int member, int64_t n, int64_t out, int64_t num_experts, const vo
     a.pairs_per_row = pairs_per_row;
     a.num_experts = uint32_t(num_experts);
     a.out_features = uint32_t(out);
+    a.wide_ids = wide_ids ? 1u : 0u;
     a.y = static_cast<uint16_t *>(y);
     switch (member) {
         case IQK_MEMBER_IQ2_KS: return launch_gemv<IQ2_KS, FLOOR != 0>(n, a, mats, st);
@@ -363,6 +366,16 @@ int iqk_gemv(int member, int64_t n, int64_t out, int64_t num_experts, const void
     const int64_t rows = pairs_per_row ? mats / pairs_per_row : 0;
     return iqk::gemv_entry<0>(member, n, out, num_experts, x, rows, streams, n_streams, sel, nullptr,
                                   pairs_per_row, mats, y, stream);
+}
+
+// The decode with 64-bit ids (sel: i64 [mats]).
+int iqk_gemv_ids64(int member, int64_t n, int64_t out, int64_t num_experts, const void *x,
+                   const void *const *streams, int n_streams, const int64_t *sel, uint32_t pairs_per_row,
+                   uint32_t mats, void *y, void *stream) {
+    const int64_t rows = pairs_per_row ? mats / pairs_per_row : 0;
+    return iqk::gemv_entry<0>(member, n, out, num_experts, x, rows, streams, n_streams,
+                              reinterpret_cast<const uint32_t *>(sel), nullptr, pairs_per_row, mats, y, stream, false,
+                              true);
 }
 
 int iqk_gemv_floor(int member, int64_t n, int64_t out, int64_t num_experts, const void *x,

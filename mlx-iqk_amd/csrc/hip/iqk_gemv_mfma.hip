@@ -78,6 +78,7 @@ struct Gemv2Args {
     uint32_t n_x_rows;
     uint32_t num_experts;
     uint32_t out_features;
+    uint32_t wide_ids;  // 1: sel holds 64-bit ids (pairs mode)
     uint16_t *y;
 };
 
@@ -942,7 +943,7 @@ void gemv_mfma_kernel(Gemv2Args a) {
     // An id beyond the stack reads expert 0 (in bounds) and writes NaN rows.
     // No early exit: a branch here would let the compiler sink the loads
     // above behind the wait for the id.
-    const uint32_t e_raw = a.sel[m0];
+    const uint32_t e_raw = MODE == kPairs ? expert_id(a.sel, m0, a.wide_ids) : a.sel[m0];
     const bool valid = e_raw < a.num_experts;  // uniform per workgroup
     const uint32_t e = valid ? e_raw : 0u;
     LaneOf<MEMBER, N> lane[R];  // rows rowg + 16 (R tile + r) + n
@@ -1065,7 +1066,7 @@ void gemv_mfma_pairs_kernel(Gemv2Args a) {
     bool valid[P];  // uniform per workgroup
 #pragma unroll
     for (int p = 0; p < P; ++p) {
-        const uint32_t e_raw = a.sel[m0 + p];
+        const uint32_t e_raw = expert_id(a.sel, m0 + p, a.wide_ids);
         valid[p] = e_raw < a.num_experts;
         e[p] = valid[p] ? e_raw : 0u;
     }
@@ -1355,8 +1356,8 @@ int pairs_per_group(uint64_t workgroups, uint32_t pairs_per_row) {
 // with union_runs the union kernel.
 int gemv_mfma_dispatch(int floor, int member, int64_t n, int64_t out, int64_t num_experts, const void *x,
                        int64_t n_x_rows, const void *const *streams, int n_streams, const uint32_t *sel,
-                       const uint32_t *toks, bool union_runs, uint32_t pairs_per_row, uint32_t mats, void *y,
-                       hipStream_t st) {
+                       bool wide_ids, const uint32_t *toks, bool union_runs, uint32_t pairs_per_row, uint32_t mats,
+                       void *y, hipStream_t st) {
     if (out % kGroupRows) return -1;
     // 32-bit offsets: every stream (the code plane is the largest, N/4 bytes a
     // row) and the activations stay below 4 GiB
@@ -1375,6 +1376,7 @@ int gemv_mfma_dispatch(int floor, int member, int64_t n, int64_t out, int64_t nu
     a.n_x_rows = uint32_t(n_x_rows);
     a.num_experts = uint32_t(num_experts);
     a.out_features = uint32_t(out);
+    a.wide_ids = wide_ids ? 1u : 0u;
     a.y = static_cast<uint16_t *>(y);
     if (!toks) {
         const uint64_t groups = uint64_t(mats) * uint64_t(out / kGroupRows);

@@ -44,6 +44,8 @@ struct RouteArgs {
     uint32_t P, E, M, ppx, n_x_rows;
 };
 
+// WIDE: 64-bit ids, of which one past 32 bits reads as 0xffffffff (no expert).
+template <bool WIDE>
 __global__ __launch_bounds__(kRouteThreads) void route_kernel(RouteArgs a) {
     __shared__ uint32_t tot[2][kRouteWaves];  // per wavefront: pairs keyed below e, keyed e
     const uint32_t e = blockIdx.x;
@@ -58,7 +60,15 @@ __global__ __launch_bounds__(kRouteThreads) void route_kernel(RouteArgs a) {
     uint32_t raw[kRoutePer];
     const auto load = [&](uint32_t base) {
 #pragma unroll
-        for (int i = 0; i < kRoutePer; ++i) raw[i] = a.ids[min(base + uint32_t(64 * i + lane), hi - 1u)];
+        for (int i = 0; i < kRoutePer; ++i) {
+            const uint32_t p = min(base + uint32_t(64 * i + lane), hi - 1u);
+            if constexpr (WIDE) {
+                const uint2_t id = reinterpret_cast<const uint2_t *>(a.ids)[p];
+                raw[i] = id.y ? 0xffffffffu : id.x;
+            } else {
+                raw[i] = a.ids[p];
+            }
+        }
     };
 
     uint32_t lt = 0, eq = 0;
@@ -112,12 +122,9 @@ __global__ __launch_bounds__(kRouteThreads) void route_kernel(RouteArgs a) {
     }
 }
 
-}  // namespace iqk
-
-extern "C" int iqk_route(const uint32_t *ids, int64_t n_pairs, int64_t num_experts, int64_t rows_per_pair,
-                         int64_t pairs_per_x_row, int64_t n_x_rows, uint32_t *group_offsets, uint32_t *x_rows,
-                         uint32_t *y_rows, void *stream) {
-    using namespace iqk;
+template <bool WIDE>
+int route_entry(const void *ids, int64_t n_pairs, int64_t num_experts, int64_t rows_per_pair, int64_t pairs_per_x_row,
+                int64_t n_x_rows, uint32_t *group_offsets, uint32_t *x_rows, uint32_t *y_rows, void *stream) {
     if (num_experts <= 0 || num_experts > kRouteMaxExperts) return IQK_ERR_ARGUMENT;
     if (n_pairs < 0 || rows_per_pair <= 0 || pairs_per_x_row <= 0 || n_x_rows < 0) return IQK_ERR_ARGUMENT;
     // each factor bounded first, so the products below cannot overflow
@@ -129,7 +136,7 @@ extern "C" int iqk_route(const uint32_t *ids, int64_t n_pairs, int64_t num_exper
     // every activation row a valid pair names lies in x
     if (n_pairs && ((n_pairs - 1) / pairs_per_x_row + 1) * rows_per_pair > n_x_rows) return IQK_ERR_ARGUMENT;
     RouteArgs a;
-    a.ids = ids;
+    a.ids = static_cast<const uint32_t *>(ids);
     a.offs = group_offsets;
     a.xr = x_rows;
     a.yr = y_rows;
@@ -138,6 +145,26 @@ extern "C" int iqk_route(const uint32_t *ids, int64_t n_pairs, int64_t num_exper
     a.M = uint32_t(rows_per_pair);
     a.ppx = uint32_t(pairs_per_x_row);
     a.n_x_rows = uint32_t(n_x_rows);
-    hipLaunchKernelGGL(route_kernel, dim3{uint32_t(num_experts)}, dim3{kRouteThreads}, 0, as_stream(stream), a);
+    hipLaunchKernelGGL(route_kernel<WIDE>, dim3{uint32_t(num_experts)}, dim3{kRouteThreads}, 0, as_stream(stream), a);
     return record_launch(hipGetLastError());
 }
+
+}  // namespace iqk
+
+extern "C" {
+
+int iqk_route(const uint32_t *ids, int64_t n_pairs, int64_t num_experts, int64_t rows_per_pair,
+              int64_t pairs_per_x_row, int64_t n_x_rows, uint32_t *group_offsets, uint32_t *x_rows, uint32_t *y_rows,
+              void *stream) {
+    return iqk::route_entry<false>(ids, n_pairs, num_experts, rows_per_pair, pairs_per_x_row, n_x_rows, group_offsets,
+                                   x_rows, y_rows, stream);
+}
+
+int iqk_route_ids64(const int64_t *ids, int64_t n_pairs, int64_t num_experts, int64_t rows_per_pair,
+                    int64_t pairs_per_x_row, int64_t n_x_rows, uint32_t *group_offsets, uint32_t *x_rows,
+                    uint32_t *y_rows, void *stream) {
+    return iqk::route_entry<true>(ids, n_pairs, num_experts, rows_per_pair, pairs_per_x_row, n_x_rows, group_offsets,
+                                  x_rows, y_rows, stream);
+}
+
+}  // extern "C"

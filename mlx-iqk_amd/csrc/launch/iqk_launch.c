@@ -25,7 +25,7 @@ static int as_i64(PyObject *o, long long *v) {
 
 /* gemv(kind, member, n, out, num_experts, x, streams, n_streams, sel,
  *      pairs_per_row, mats, y, stream): kind 0 iqk_gemv, 1 iqk_gemv_floor,
- * 2 iqk_gemv_floor_grid; streams is the address of the stream pointer array. */
+ * 2 iqk_gemv_floor_grid, 3 iqk_gemv_ids64; streams is the address of the stream pointer array. */
 static PyObject *gemv(PyObject *self, PyObject *const *args, Py_ssize_t nargs) {
     (void)self;
     if (nargs != 13) {
@@ -42,6 +42,13 @@ static PyObject *gemv(PyObject *self, PyObject *const *args, Py_ssize_t nargs) {
         PyErr_SetString(PyExc_OverflowError, "gemv: member, stream count, pairs per row or pair count out of range");
         return NULL;
     }
+    if (v[0] == 3) {
+        const int rc = iqk_gemv_ids64((int)v[1], (int64_t)v[2], (int64_t)v[3], (int64_t)v[4],
+                                      (const void *)(uintptr_t)v[5], (const void *const *)(uintptr_t)v[6], (int)v[7],
+                                      (const int64_t *)(uintptr_t)v[8], (uint32_t)v[9], (uint32_t)v[10],
+                                      (void *)(uintptr_t)v[11], (void *)(uintptr_t)v[12]);
+        return PyLong_FromLong(rc);
+    }
     int (*fn)(int, int64_t, int64_t, int64_t, const void *, const void *const *, int, const uint32_t *, uint32_t,
               uint32_t, void *, void *) = v[0] == 1 ? iqk_gemv_floor : v[0] == 2 ? iqk_gemv_floor_grid : iqk_gemv;
     const int rc = fn((int)v[1], (int64_t)v[2], (int64_t)v[3], (int64_t)v[4], (const void *)(uintptr_t)v[5],
@@ -57,7 +64,7 @@ static PyObject *source_hash(PyObject *self, PyObject *unused) {
 }
 
 static PyMethodDef methods[] = {
-    {"gemv", (PyCFunction)(void (*)(void))gemv, METH_FASTCALL, "iqk_gemv / _floor / _floor_grid"},
+    {"gemv", (PyCFunction)(void (*)(void))gemv, METH_FASTCALL, "iqk_gemv / _floor / _floor_grid / _ids64"},
     {"source_hash", source_hash, METH_NOARGS, "digest of the kernel sources this binding was built with"},
     {NULL, NULL, 0, NULL},
 };

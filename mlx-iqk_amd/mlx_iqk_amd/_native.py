@@ -13,7 +13,7 @@ from pathlib import Path
 from . import build
 from .build import HIP_LIB, LAUNCH_EXT
 
-ABI_VERSION = 5
+ABI_VERSION = 6
 
 OK, ERR_MEMBER, ERR_GEOMETRY, ERR_ARGUMENT, ERR_LAUNCH = 0, 1, 2, 3, 4
 _CODES = {ERR_MEMBER: "unknown member", ERR_GEOMETRY: "unsized geometry",
@@ -33,6 +33,8 @@ SIGNATURES = {
     "iqk_check_dequant_geometry": (c_int, [c_int, c_int64, c_int64]),
     "iqk_gemv": (c_int, [c_int, c_int64, c_int64, c_int64, c_void_p, ctypes.POINTER(c_void_p), c_int,
                          c_void_p, c_uint32, c_uint32, c_void_p, c_void_p]),
+    "iqk_gemv_ids64": (c_int, [c_int, c_int64, c_int64, c_int64, c_void_p, ctypes.POINTER(c_void_p), c_int,
+                               c_void_p, c_uint32, c_uint32, c_void_p, c_void_p]),
     "iqk_gemv_floor": (c_int, [c_int, c_int64, c_int64, c_int64, c_void_p, ctypes.POINTER(c_void_p), c_int,
                                c_void_p, c_uint32, c_uint32, c_void_p, c_void_p]),
     "iqk_gemv_floor_grid": (c_int, [c_int, c_int64, c_int64, c_int64, c_void_p, ctypes.POINTER(c_void_p), c_int,
@@ -53,6 +55,8 @@ SIGNATURES = {
                                  c_void_p, c_void_p, c_void_p, c_void_p, c_void_p]),
     "iqk_route": (c_int, [c_void_p, c_int64, c_int64, c_int64, c_int64, c_int64, c_void_p, c_void_p, c_void_p,
                           c_void_p]),
+    "iqk_route_ids64": (c_int, [c_void_p, c_int64, c_int64, c_int64, c_int64, c_int64, c_void_p, c_void_p, c_void_p,
+                                c_void_p]),
     "iqk_pack": (c_int, [c_int, c_int64, c_int64, c_void_p, ctypes.POINTER(c_void_p), c_int, c_void_p]),
     "iqk_fused_gemm": (c_int, [c_int, c_int64, c_int64, c_int64, c_void_p, c_int64, ctypes.POINTER(c_void_p),
                                c_int, c_int64, c_int64, c_void_p, c_void_p, c_void_p, c_int64, c_void_p, c_void_p]),

@@ -196,8 +196,8 @@ def gemv(member: str, x: torch.Tensor, streams: list[torch.Tensor], sel: torch.T
 
 def _gemv_launch(kind: int, member: str, n: int, out_features: int, num_experts: int, xp: int, ptrs, n_streams: int,
                  sp: int, pairs_per_row: int, mats: int, yp: int, stream: int) -> None:
-    """The launches of :func:`gemv` (kind 0 decode, 1 floor, 2 grid floor) on
-    operands already checked: device addresses of x, sel and y, the streams'
+    """The launches of :func:`gemv` (kind 0 decode, 1 floor, 2 grid floor, 3
+    decode with 64-bit ids) on operands already checked: device addresses of x, sel and y, the streams'
     pointer array.  gridDim.y carries the pair index, so the pairs go in
     chunks that keep whole activation rows together."""
     if not 0 < pairs_per_row <= 65535:  # one launch takes at most 65535 pairs
@@ -207,24 +207,27 @@ def _gemv_launch(kind: int, member: str, n: int, out_features: int, num_experts:
     ptrs_addr = ctypes.addressof(ptrs)
     limit = (65535 // pairs_per_row) * pairs_per_row
     mid = _native.MEMBER_IDS[member]
+    id_bytes = 8 if kind == 3 else 4
     for m0 in range(0, mats, limit):
         cnt = min(limit, mats - m0)
         args = (mid, n, out_features, num_experts, xp + (m0 // pairs_per_row) * n * 2, ptrs_addr, n_streams,
-                sp + 4 * m0, pairs_per_row, cnt, yp + m0 * out_features * 2, stream)
+                sp + id_bytes * m0, pairs_per_row, cnt, yp + m0 * out_features * 2, stream)
         if fast is not None:
             rc = fast.gemv(kind, *args)
         else:
-            fn = (lib.iqk_gemv, lib.iqk_gemv_floor, lib.iqk_gemv_floor_grid)[kind]
+            fn = (lib.iqk_gemv, lib.iqk_gemv_floor, lib.iqk_gemv_floor_grid, lib.iqk_gemv_ids64)[kind]
             rc = fn(*args[:5], ptrs, *args[6:])
         if rc:  # the message is formatted only for a failure
-            _native.check(rc, f"iqk_gemv{'_floor' if kind else ''}({member}, {n}x{out_features})")
+            _native.check(rc, f"iqk_gemv{'_floor' if kind in (1, 2) else ''}({member}, {n}x{out_features})")
 
 
 def gemv_checked(member: str, x: torch.Tensor, streams: "CheckedStreams", sel: torch.Tensor, rows: int, mats: int,
-                 out: torch.Tensor, num_experts: int, out_features: int) -> None:
+                 out: torch.Tensor, num_experts: int, out_features: int, wide: bool = False) -> None:
     """The decode GEMV into ``out`` for operands the caller has checked: x
     fp16 and contiguous with ``rows`` rows of the streams' width, sel int32
-    and contiguous with ``mats`` ids, out fp16 with ``mats x out_features``
+    (``wide``: int64, which the kernel reads itself: without the three
+    launches that clamped and narrowed the ids an eager call takes 8.4 us, not
+    23.5) and contiguous with ``mats`` ids, out fp16 with ``mats x out_features``
     elements, all on the streams' GPU, ``streams.gemv_ok`` and
     ``mats % rows == 0``.  (The switch module's eager decode path: it skips
     the reshapes and repeated checks of :func:`gemv`.)"""
@@ -232,14 +235,15 @@ def gemv_checked(member: str, x: torch.Tensor, streams: "CheckedStreams", sel: t
         return
     stream = (_raw_stream(streams.device_index) if _raw_stream is not None
               else torch.cuda.current_stream(streams.device).cuda_stream)
+    kind = 3 if wide else 0
     fast = _native.launcher()
     if fast is not None and mats <= 65535:  # one launch: the binding's call with nothing else around it
-        rc = fast.gemv(0, _native.MEMBER_IDS[member], streams.key[3], out_features, num_experts, x.data_ptr(),
+        rc = fast.gemv(kind, _native.MEMBER_IDS[member], streams.key[3], out_features, num_experts, x.data_ptr(),
                        streams.ptrs_addr, streams.count, sel.data_ptr(), mats // rows, mats, out.data_ptr(), stream)
         if rc:
             _native.check(rc, f"iqk_gemv({member}, {streams.key[3]}x{out_features})")
         return
-    _gemv_launch(0, member, streams.key[3], out_features, num_experts, x.data_ptr(), streams.ptrs, streams.count,
+    _gemv_launch(kind, member, streams.key[3], out_features, num_experts, x.data_ptr(), streams.ptrs, streams.count,
                  sel.data_ptr(), mats // rows, mats, out.data_ptr(), stream)
 
 
@@ -487,6 +491,13 @@ def route(ids: torch.Tensor, num_experts: int, rows_per_pair: int = 1, pairs_per
     order is stable (pairs keep their order within an expert).
     """
     _require_cuda(ids, "ids", (torch.int32, torch.uint32))
+    return route_ids(ids, num_experts, rows_per_pair, pairs_per_x_row, n_x_rows)
+
+
+def route_ids(ids: torch.Tensor, num_experts: int, rows_per_pair: int = 1, pairs_per_x_row: int = 1,
+              n_x_rows: int | None = None) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
+    """:func:`route` for int64 ids too (the switch module's prefill)."""
+    _require_cuda(ids, "ids", (torch.int32, torch.uint32, torch.int64))
     if ids.dim() != 1:
         raise IqkKernelError("ids must be [pairs]")
     E, P, M, ppx = int(num_experts), int(ids.numel()), int(rows_per_pair), int(pairs_per_x_row)
@@ -498,8 +509,10 @@ def route(ids: torch.Tensor, num_experts: int, rows_per_pair: int = 1, pairs_per
     offs = torch.empty(E + 1, dtype=torch.int32, device=ids.device)
     x_rows = torch.empty(P * M, dtype=torch.int32, device=ids.device)
     y_rows = torch.empty(P * M, dtype=torch.int32, device=ids.device)
-    rc = _native.load().iqk_route(ids.data_ptr(), P, E, M, ppx, rows, offs.data_ptr(), x_rows.data_ptr(),
-                                  y_rows.data_ptr(), _stream_ptr(ids.device))
+    lib = _native.load()
+    fn = lib.iqk_route_ids64 if ids.dtype == torch.int64 else lib.iqk_route
+    rc = fn(ids.data_ptr(), P, E, M, ppx, rows, offs.data_ptr(), x_rows.data_ptr(), y_rows.data_ptr(),
+            _stream_ptr(ids.device))
     if rc:
         _native.check(rc, f"iqk_route(P={P}, E={E}, M={M})")
     return offs, x_rows, y_rows

@@ -35,6 +35,9 @@ from .format import IQ2NL_VALUES, check_member, component_shapes
 from .iq1grid import grid_values
 from .kernels import IqkKernelError, check_dequant_geometry, check_gemv_geometry, stream_dtypes
 
+_KERNEL_IDS = {torch.int32: False, torch.int64: True}
+"""Id types the decode and the route kernels read as they are: whether wide."""
+
 DECODE_MAT_LIMIT = 63
 """Token-expert pairs at or below which the decode GEMV serves
 (reference: src/mlx_iqk/nn.py:49-54)."""
@@ -226,18 +229,19 @@ class IqkSwitchLinear(torch.nn.Module):
         """Fused GEMV over the selected experts; valid for any pair count
         (reference: src/mlx_iqk/nn.py:240-271)."""
         chk = self._checked()
-        # Operands already in the kernel's layout (fp16 contiguous x, int32
-        # contiguous ids, on the streams' GPU) launch without a reshape and
+        # Operands already in the kernel's layout (fp16 contiguous x, int32 or
+        # int64 contiguous ids, on the streams' GPU) launch without a reshape and
         # with the output allocated in its final shape: the eager decode's
         # host time is mostly such tensor operations.
-        if (x.dtype == torch.float16 and indices.dtype == torch.int32 and chk.gemv_ok
+        wide = _KERNEL_IDS.get(indices.dtype)
+        if (x.dtype == torch.float16 and wide is not None and chk.gemv_ok
                 and x.is_contiguous() and indices.is_contiguous() and x.shape[-1] == self.in_features
                 and x.get_device() == chk.device_index and indices.get_device() == chk.device_index):
             mats, rows = indices.numel(), x.numel() // self.in_features
             if rows > 0 and mats % rows == 0:
                 out = torch.empty((*indices.shape, 1, self.out_features), dtype=torch.float16, device=chk.device)
                 kernels.gemv_checked(self.member, x, chk, indices, rows, mats, out, self.num_experts,
-                                     self.out_features)
+                                     self.out_features, wide)
                 return out
         xt = x.reshape(-1, self.in_features)
         if xt.dtype != torch.float16 or not xt.is_contiguous():
@@ -365,8 +369,10 @@ class IqkSwitchLinear(torch.nn.Module):
         while lead < len(batch) and pad[lead] == batch[lead]:
             lead += 1
         if all(d == 1 for d in pad[lead:]) and E <= kernels.ROUTE_MAX_EXPERTS:
-            ids = self._device_ids(indices.to(device).broadcast_to(batch))
-            return kernels.route(ids, E, M, math.prod(batch[lead:]), n_x_rows)
+            ids = indices.to(device).broadcast_to(batch).reshape(-1)
+            if ids.dtype not in _KERNEL_IDS or not ids.is_contiguous():
+                ids = self._device_ids(ids)
+            return kernels.route_ids(ids, E, M, math.prod(batch[lead:]), n_x_rows)
         xidx = torch.arange(math.prod(xbatch), device=device).reshape(xbatch).broadcast_to(batch).reshape(-1)
         raw = indices.to(device=device, dtype=torch.int64).broadcast_to(batch).reshape(-1)
         valid = (raw >= 0) & (raw < E)
