@@ -87,47 +87,81 @@ struct FusedArgs {
     uint32_t n_groups, n_slots, n_x_rows;
 };
 
-struct FusedScan {
-    TileScan many;
-    uint32_t wave[kFusedWaves], group, mtile;
+// How a launch cuts a group's slots into tiles.
+enum TileCut : int {
+    kCut64 = 0,    // 64-slot tiles, the last one partial
+    kCutWide = 1,  // 128-slot tiles, the last one if it holds more than 64
+    kCutRest = 2,  // what kCutWide leaves: one tile of at most 64 slots, or none
 };
 
-// The (group, M-tile) of an XCD's nth tile: XCD x takes tiles x ceil(T / 8) ..
-// of the list's T.  False (uniformly) past its share.  Up to a group a thread,
-// the sizes are loaded and scanned once, for T and the tile both.
-__device__ __forceinline__ bool claim_mtile(const uint32_t *offs, uint32_t n_groups, uint32_t xcd, uint32_t nth,
-                                            FusedScan &ts, uint32_t &group, uint32_t &mtile) {
-    if (n_groups > uint32_t(kFusedThreads)) {  // uniform
-        const uint32_t tiles = count_mtiles<kFusedBM, kFusedThreads>(offs, n_groups, ts.many);
-        const uint32_t per_xcd = (tiles + 7) / 8, tile = xcd * per_xcd + nth;
-        if (nth >= per_xcd || tile >= tiles) return false;
-        return find_mtile<kFusedBM, kFusedThreads>(offs, n_groups, tile, ts.many, group, mtile);
-    }
+constexpr uint32_t kWideBM = 128;  // slots of a wide tile
+
+template <int CUT>
+__device__ __forceinline__ uint32_t tiles_of(uint32_t slots) {
+    const uint32_t rest = slots % kWideBM;
+    if constexpr (CUT == kCut64) return (slots + kFusedBM - 1) / kFusedBM;
+    if constexpr (CUT == kCutWide) return slots / kWideBM + (rest > uint32_t(kFusedBM) ? 1u : 0u);
+    return rest != 0 && rest <= uint32_t(kFusedBM) ? 1u : 0u;
+}
+
+struct FusedScan {
+    uint32_t wave[8], group, tile;
+};
+
+// The group of an XCD's nth tile, and the tile's number within it: XCD x takes
+// tiles x ceil(T / 8) .. of the list's T, in group order.  False (uniformly)
+// past its share.  Up to a group a thread, the sizes are loaded and scanned
+// once, for T and the tile both.  share: ceil(T / 8).
+template <int CUT, int THREADS>
+__device__ __forceinline__ bool claim_tile(const uint32_t *offs, uint32_t n_groups, uint32_t xcd, uint32_t nth,
+                                           FusedScan &ts, uint32_t &group, uint32_t &mtile, uint32_t &share) {
     const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const uint32_t cnt = tid < n_groups ? (offs[tid + 1] - offs[tid] + kFusedBM - 1) / kFusedBM : 0u;
-    uint32_t incl = cnt;
+    const auto tiles_at = [&](uint32_t g) { return g < n_groups ? tiles_of<CUT>(offs[g + 1] - offs[g]) : 0u; };
+    const bool once = n_groups <= uint32_t(THREADS);  // uniform
+    uint32_t total = 0;
+    if (!once) {
+        uint32_t cnt = 0;
+        for (uint32_t g = tid; g < n_groups; g += THREADS) cnt += tiles_at(g);
 #pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-        const uint32_t up = __shfl_up(incl, off, 64);
-        if (lane >= uint32_t(off)) incl += up;
-    }
-    if (lane == 63) ts.wave[wave] = incl;
-    __syncthreads();
-    uint32_t tiles = 0, before = 0;
+        for (int off = 32; off > 0; off >>= 1) cnt += __shfl_xor(cnt, off, 64);
+        if (lane == 0) ts.wave[wave] = cnt;
+        __syncthreads();
 #pragma unroll
-    for (uint32_t w = 0; w < uint32_t(kFusedWaves); ++w) {
-        before += w < wave ? ts.wave[w] : 0u;
-        tiles += ts.wave[w];
+        for (int w = 0; w < THREADS / 64; ++w) total += ts.wave[w];
+        __syncthreads();  // the rounds below rewrite the totals
     }
-    const uint32_t per_xcd = (tiles + 7) / 8, tile = xcd * per_xcd + nth, excl = before + incl - cnt;
-    if (nth >= per_xcd || tile >= tiles) return false;  // uniform
-    if (tile - excl < cnt) {  // exactly one thread's
-        ts.group = tid;
-        ts.mtile = tile - excl;
+    uint32_t carry = 0, tile = 0;
+    for (uint32_t base = 0; base < n_groups; base += THREADS) {
+        const uint32_t cnt = tiles_at(base + tid);
+        uint32_t incl = cnt;
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+            const uint32_t up = __shfl_up(incl, off, 64);
+            if (lane >= uint32_t(off)) incl += up;
+        }
+        if (lane == 63) ts.wave[wave] = incl;
+        __syncthreads();
+        uint32_t sum = 0, before = 0;
+#pragma unroll
+        for (uint32_t w = 0; w < uint32_t(THREADS / 64); ++w) {
+            before += w < wave ? ts.wave[w] : 0u;
+            sum += ts.wave[w];
+        }
+        if (once) total = sum;
+        const uint32_t excl = carry + before + incl - cnt;
+        share = (total + 7) / 8;
+        tile = xcd * share + nth;
+        if (nth >= share || tile >= total) return false;  // uniform
+        if (tile - excl < cnt) {  // one thread's, of all rounds
+            ts.group = base + tid;
+            ts.tile = tile - excl;
+        }
+        carry += sum;
+        __syncthreads();
+        if (tile < carry) break;  // uniform: found
     }
-    __syncthreads();
-    group = ts.group;
-    mtile = ts.mtile;
+    group = __builtin_amdgcn_readfirstlane(ts.group);  // uniform (read from LDS): the stream bases stay scalar
+    mtile = __builtin_amdgcn_readfirstlane(ts.tile);
     return true;
 }
 
@@ -690,10 +724,8 @@ void fused_gemm_kernel(FusedArgs a) {
     const int tid = threadIdx.x;
     const uint32_t ncb = (a.N + kFusedBN - 1) / kFusedBN;  // column blocks
     const uint32_t xcd = blockIdx.x & 7u, j = blockIdx.x >> 3, cblock = j % ncb;
-    uint32_t g, mtile;
-    if (!claim_mtile(a.offs, a.n_groups, xcd, j / ncb, ts, g, mtile)) return;  // surplus block (uniform)
-    g = __builtin_amdgcn_readfirstlane(g);  // uniform (read from LDS): the stream bases stay scalar
-    mtile = __builtin_amdgcn_readfirstlane(mtile);
+    uint32_t g, mtile, share;
+    if (!claim_tile<kCut64, kFusedThreads>(a.offs, a.n_groups, xcd, j / ncb, ts, g, mtile, share)) return;  // surplus
 
     // Offsets and row indices are device data: a slot outside [0, n_slots)
     // is never stored, a row outside x is never read (its output row is NaN),
@@ -985,16 +1017,342 @@ void fused_gemm_kernel(FusedArgs a) {
         run_steps(std::integral_constant<int, 2>{});
 }
 
-template <int MEMBER>
-int launch_fused(int64_t k, const FusedArgs &a, uint32_t n_slots, hipStream_t st) {
-    const uint64_t mtiles = (uint64_t(n_slots) + kFusedBM - 1) / kFusedBM + uint64_t(a.n_groups);
-    const uint64_t blocks = (mtiles + 7) / 8 * 8 * ((a.N + kFusedBN - 1) / kFusedBN);
+// ---- wide tiles -------------------------------------------------------------------
+
+constexpr int kWideThreads = 256;
+constexpr int kWideBN = 256;  // weight rows per block: 64 a wavefront
+
+// One lane's weights of one row (ln) in steps of 128, as the 64-slot tile
+// takes them: lane group kg the sub-blocks 2kg, 2kg + 1 of a step (IQ1_S_R4, whose
+// steps go in pairs: elements 256p + 128kg + 64j .. +63 of pair p in its step
+// j).  Code words a step ahead; scales of four steps at once (the IQ2 members).
+template <int MEMBER, int K>
+struct WideLane {
+    static constexpr bool IQ1 = MEMBER == IQ1_S_R4, KS = MEMBER == IQ2_KS;
+    uint4_t q;   // IQ2: a step's code words; IQ1_S_R4: a pair's index words
+    uint2_t h;   // IQ1_S_R4: a pair's qh words
+
+    __device__ __forceinline__ void load(const FewPlanes<MEMBER, K> &pl, uint32_t row, int kg, int s) {
+        using P = FewPlanes<MEMBER, K>;
+        if constexpr (IQ1) {
+            q = buffer_u4(pl.p[0], row * P::ROW[0] + 16 * kg, 32 * (s >> 1));
+            h = __builtin_amdgcn_raw_buffer_load_b64(pl.p[1], row * P::ROW[1] + 8 * kg, 16 * (s >> 1), 0);
+        } else {
+            q = buffer_u4(pl.p[0], row * P::ROW[0] + 16 * kg, 32 * s);
+        }
+    }
+};
+
+template <int MEMBER, int K>
+struct WideScales {
+    uint4_t sc;       // IQ2_KS: scl bytes of steps 4p .. 4p+3 (x, y); IQ2_K: scl words
+    uint32_t e0, e1;  // IQ2_KS: sch, sex of super-blocks 2p, 2p+1; IQ2_K: sex of the four steps, dv
+
+    __device__ __forceinline__ void load(const FewPlanes<MEMBER, K> &pl, uint32_t row, int p) {
+        using P = FewPlanes<MEMBER, K>;
+        if constexpr (MEMBER == IQ2_KS) {
+            const uint2_t v = __builtin_amdgcn_raw_buffer_load_b64(pl.p[1], row * P::ROW[1], 8 * p, 0);
+            sc.x = v.x;
+            sc.y = v.y;
+            e0 = __builtin_amdgcn_raw_buffer_load_b16(pl.p[2], row * P::ROW[2], 2 * p, 0);
+            e1 = __builtin_amdgcn_raw_buffer_load_b16(pl.p[3], row * P::ROW[3], 2 * p, 0);
+        } else if constexpr (MEMBER == IQ2_K) {
+            sc = buffer_u4(pl.p[1], row * P::ROW[1], 16 * p);
+            e0 = __builtin_amdgcn_raw_buffer_load_b32(pl.p[2], row * P::ROW[2], 4 * p, 0);
+            e1 = __builtin_amdgcn_raw_buffer_load_b32(pl.p[3], row * P::ROW[3], 4 * p, 0);
+        }
+    }
+    // the tables of step 4p + i, lane group kg
+    __device__ __forceinline__ void tables(int i, int kg, const uint2_t *ptab, Pool *p) const {
+        if constexpr (MEMBER == IQ2_KS) {
+            const uint32_t scl = (i < 2 ? sc.x : sc.y) >> (16 * (i & 1) + 8 * kg);
+            const int bit = 8 * (i >> 1) + 4 * (i & 1) + 2 * kg;
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+                const uint32_t e =
+                    ((scl >> (4 * t)) & 15u) | (((e0 >> (bit + t)) & 1u) << 4) | (((e1 >> (bit + t)) & 1u) << 5);
+                const uint2_t v = ptab[e];
+                p[2 * t] = {v.x, v.y};
+                p[2 * t + 1] = p[2 * t];
+            }
+        } else if constexpr (MEMBER == IQ2_K) {
+            iq2k_pools((sc[i] >> (16 * kg)) & 0xffffu, (e0 >> (8 * i + 4 * kg)) & 15u,
+                       half_of_bits((e1 >> (16 * (i >> 1))) & 0xffffu), ptab, p);
+        }
+    }
+};
+
+// Tiles of up to 128 slots, for calls whose experts have many: four wavefronts
+// of 64 weight rows, each for all the tile's slots, so an activation fragment
+// read from LDS feeds two MFMAs and a decoded weight four (the 64-slot tile's:
+// one and two).  128 of a wavefront's 256 VGPRs are accumulators; two blocks a
+// CU, one wavefront of each a SIMD: one's VALU work runs under the other's
+// MFMAs (290 VALU a step of 64 MFMAs of 32 cycles).  The block's scales
+// come straight from their planes, four steps at a time, and the activations
+// (64 rows at a time, half a step ahead) are the only thing staged.  Groups
+// are cut into 128-slot tiles, a last one of more than 64 slots among them;
+// what is left (at most 64 slots a group) goes last in the list, so the short
+// tiles fill the end of the launch.  It reaches 0.9 to 1.08 PFLOP/s where an
+// 8192-wide fp16 library product reaches 1.08 on this card (the clock its
+// power allows).
+template <int MEMBER, int K>
+__global__ __launch_bounds__(kWideThreads) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void wide_gemm_kernel(FusedArgs a) {
+    constexpr bool IQ1 = MEMBER == IQ1_S_R4;
+    constexpr int STEPS = K / kFusedKS;
+    static_assert(STEPS % 4 == 0, "whole groups of scales");
+    __shared__ FusedScan ts;
+    __shared__ uint32_t slot_dst[kWideBM];
+    __shared__ uint2_t ptab[MEMBER == IQ2_K ? 32 : IQ1 ? 16 : 64];
+    __shared__ __attribute__((aligned(16))) uint16_t codes[IQ1 ? IQK_IQ1S_GRID_SIZE : 8];
+    __shared__ __attribute__((aligned(16))) uint8_t xs[2][kWideBM * kXStride];
+
+    const int tid = threadIdx.x;
+    const uint32_t ncb = (a.N + kWideBN - 1) / kWideBN;
+    // the wide tiles first (the long ones), then the rests
+    const uint32_t xcd = blockIdx.x & 7u, nth = (blockIdx.x >> 3) / ncb, cblock = (blockIdx.x >> 3) % ncb;
+    uint32_t g, mtile, share;
+    if (!claim_tile<kCutWide, kWideThreads>(a.offs, a.n_groups, xcd, nth, ts, g, mtile, share)) {
+        if (nth < share) return;  // uniform
+        __syncthreads();          // the first claim's totals have been read
+        const uint32_t wide = share;
+        if (!claim_tile<kCutRest, kWideThreads>(a.offs, a.n_groups, xcd, nth - wide, ts, g, mtile, share)) return;
+        mtile = (a.offs[g + 1] - a.offs[g]) / kWideBM;
+    }
+    const uint32_t gend = min(a.offs[g + 1], a.n_slots);
+    const uint32_t m0 = a.offs[g] + mtile * kWideBM;
+    const uint32_t n0 = cblock * kWideBN;
+    const size_t row0 = size_t(g) * a.out_rows + a.row_start + n0;
+    const FewPlanes<MEMBER, K> planes(a, row0);
+
+    const int wave = tid >> 6, l = tid & 63, ln = l & 31, kg = l >> 5;
+    const uint32_t wrow = uint32_t(64 * wave + ln);  // and wrow + 32
+    WideLane<MEMBER, K> cur[2], nxt[2];
+    WideScales<MEMBER, K> sc[2], scn[2];
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+        cur[b].load(planes, wrow + 32 * b, kg, 0);
+        if constexpr (!IQ1) sc[b].load(planes, wrow + 32 * b, 0);
+    }
+    if constexpr (MEMBER == IQ2_K) {
+        if (tid < 32) ptab[tid] = reinterpret_cast<const uint2_t *>(kIq2kProducts.w)[tid];
+    } else if constexpr (IQ1) {
+        if (tid < 16) ptab[tid] = kIq1Pools.p[tid];
+        static_assert(IQK_IQ1S_GRID_SIZE == 8 * kWideThreads, "eight grid entries a thread");
+        reinterpret_cast<uint4_t *>(codes)[tid] = reinterpret_cast<const uint4_t *>(iqk_iq1s_grid_codes)[tid];
+    } else {
+        if (tid < 64) ptab[tid] = kIq2ksPools.p[tid];
+    }
+    // staging: thread t moves 16-byte chunk t % 16 of slot rows t / 16 + 16 i; a
+    // row past the tile's last slot, or past x, lies past x's buffer: zeros
+    const int xrow = tid / kXChunks, xchunk = tid % kXChunks;
+    constexpr int ROWS_A_PASS = kWideThreads / kXChunks, PASSES = int(kWideBM) / ROWS_A_PASS;
+    const uint32_t xbytes = a.n_x_rows * uint32_t(2 * K);
+    const __amdgpu_buffer_rsrc_t xbuf = buffer_of(a.x, xbytes);
+    uint32_t xoff[PASSES];
+#pragma unroll
+    for (int i = 0; i < PASSES; ++i) {
+        const uint32_t xp = m0 + uint32_t(xrow + ROWS_A_PASS * i);
+        const bool live = xp < gend;
+        const uint32_t row = live ? a.xr[xp] : a.n_x_rows;
+        const bool xv = row < a.n_x_rows;  // else its output is NaN
+        xoff[i] = xv ? row * uint32_t(2 * K) + uint32_t(16 * xchunk) + (IQ1 && xchunk >= 8 ? 128u : 0u) : xbytes;
+        if (xchunk == 0) {
+            uint32_t dst = kNoStore;
+            if (live) {
+                const uint32_t yrow = a.yr ? a.yr[xp] : xp;
+                if (yrow < a.n_slots) dst = yrow | (xv ? 0x80000000u : 0u);
+            }
+            slot_dst[xrow + ROWS_A_PASS * i] = dst;
+        }
+    }
+    constexpr int BATCH = PASSES / 2;  // rows go in two batches of 64
+    const auto load_x = [&](int s, int b, uint4_t (&v)[BATCH]) {
+        const uint32_t off = IQ1 ? uint32_t(512 * (s >> 1) + 128 * (s & 1)) : uint32_t(256 * s);
+#pragma unroll
+        for (int i = 0; i < BATCH; ++i) v[i] = buffer_u4(xbuf, xoff[BATCH * b + i], off);
+    };
+    const auto store_x = [&](int buf, int b, const uint4_t (&v)[BATCH]) {
+        uint8_t *dst = xs[buf] + (xrow + 64 * b) * kXStride + 16 * xchunk;
+#pragma unroll
+        for (int i = 0; i < BATCH; ++i)
+            *reinterpret_cast<uint4_t *>(dst + ROWS_A_PASS * kXStride * i) =
+                uint4_t{perm(v[i].z, v[i].x, 0x05040100u), perm(v[i].z, v[i].x, 0x07060302u),
+                        perm(v[i].w, v[i].y, 0x05040100u), perm(v[i].w, v[i].y, 0x07060302u)};
+    };
+    uint4_t xv[BATCH];
+    load_x(0, 0, xv);
+    store_x(0, 0, xv);
+    if (gend - m0 > uint32_t(kFusedBM)) {  // uniform
+        load_x(0, 1, xv);
+        store_x(0, 1, xv);
+    }
+    __syncthreads();
+
+    // MB blocks of 32 slots
+    const auto run = [&](auto blocks) {
+        constexpr int MB = decltype(blocks)::value;
+
+        float16_t acc[2][MB];
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+#pragma unroll
+            for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) acc[b][mb][r] = 0.f;
+        const uint8_t *const abase = xs[0] + ln * kXStride + 128 * kg;
+        // step 4p + i, the code words in `now`, the next step's to `then`
+        const auto step = [&](int p, int i, const WideLane<MEMBER, K> (&now)[2], WideLane<MEMBER, K> (&then)[2]) {
+            const int s = 4 * p + i;
+            const bool more = s + 1 < STEPS;
+            if (more) load_x(s + 1, 0, xv);
+            if (more && (!IQ1 || (i & 1))) {
+#pragma unroll
+                for (int b = 0; b < 2; ++b) then[b].load(planes, wrow + 32 * b, kg, s + 1);
+            }
+            if (!IQ1 && i == 0 && p + 1 < STEPS / 4) {
+#pragma unroll
+                for (int b = 0; b < 2; ++b) scn[b].load(planes, wrow + 32 * b, p + 1);
+            }
+            Pool pool[2][4];
+            uint32_t words[2][4];
+#pragma unroll
+            for (int b = 0; b < 2; ++b) {
+                if constexpr (IQ1) {
+                    const uint32_t hw = i & 1 ? now[b].h.y : now[b].h.x;
+#pragma unroll
+                    for (int t = 0; t < 2; ++t) {  // blocks 2j, 2j + 1 of the pair
+                        const uint32_t qw = now[b].q[2 * (i & 1) + t], h = (hw >> (16 * t)) & 0xffffu;
+                        const uint2_t v = ptab[(h >> 12) & 15u];
+                        pool[b][2 * t] = {v.x, v.y};
+                        pool[b][2 * t + 1] = pool[b][2 * t];
+                        uint32_t c[4];
+#pragma unroll
+                        for (int k = 0; k < 4; ++k) c[k] = codes[((qw >> (8 * k)) & 0xffu) | (((h >> (3 * k)) & 7u) << 8)];
+                        words[b][2 * t] = perm(c[1], c[0], 0x05040100u);
+                        words[b][2 * t + 1] = perm(c[3], c[2], 0x05040100u);
+                    }
+                } else {
+                    sc[b].tables(i, kg, ptab, pool[b]);
+#pragma unroll
+                    for (int w = 0; w < 4; ++w) words[b][w] = now[b].q[w];
+                }
+            }
+            const uint8_t *const ab = abase + (s & 1) * int(sizeof(xs[0]));
+#pragma unroll
+            for (int w = 0; w < 4; ++w) {
+                uint32_t bw[2][8];
+#pragma unroll
+                for (int b = 0; b < 2; ++b) expand_word_paired(words[b][w], pool[b][w], bw[b]);
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    half8_t af[MB];
+#pragma unroll
+                    for (int mb = 0; mb < MB; ++mb)
+                        af[mb] = __builtin_bit_cast(
+                            half8_t, *reinterpret_cast<const uint4_t *>(ab + 32 * mb * kXStride + 32 * w + 16 * h));
+#pragma unroll
+                    for (int b = 0; b < 2; ++b) {
+                        const half8_t bf = __builtin_bit_cast(half8_t, uint4_t{bw[b][h], bw[b][2 + h], bw[b][4 + h], bw[b][6 + h]});
+#pragma unroll
+                        for (int mb = 0; mb < MB; ++mb)
+                            acc[b][mb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[mb], bf, acc[b][mb], 0, 0, 0);
+                    }
+                }
+                if (w == 1 && more) {
+                    store_x((s + 1) & 1, 0, xv);
+                    if (MB > 2) load_x(s + 1, 1, xv);
+                }
+            }
+            if (MB > 2 && more) store_x((s + 1) & 1, 1, xv);
+            if (!IQ1 && i == 3) {
+#pragma unroll
+                for (int b = 0; b < 2; ++b) sc[b] = scn[b];
+            }
+            __syncthreads();
+        };
+#pragma unroll 1
+        for (int p = 0; p < STEPS / 4; ++p) {
+            if constexpr (IQ1) {  // a pair's words serve two steps
+                step(p, 0, cur, nxt);
+                step(p, 1, cur, nxt);
+                step(p, 2, nxt, cur);
+                step(p, 3, nxt, cur);
+            } else {
+                step(p, 0, cur, nxt);
+                step(p, 1, nxt, cur);
+                step(p, 2, cur, nxt);
+                step(p, 3, nxt, cur);
+            }
+        }
+
+#pragma unroll
+        for (int b = 0; b < 2; ++b) {
+            const uint32_t col = n0 + wrow + 32 * b;
+            if (col >= a.N) continue;
+            float d = 1.f;
+            if constexpr (MEMBER == IQ2_KS) d = float(half_of_bits(static_cast<const uint16_t *>(a.s4)[row0 + wrow + 32 * b]));
+            if constexpr (IQ1) d = float(half_of_bits(static_cast<const uint16_t *>(a.s2)[row0 + wrow + 32 * b]));
+#pragma unroll
+            for (int mb = 0; mb < MB; ++mb) {
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    const uint32_t dst = slot_dst[32 * mb + 8 * (r >> 2) + 4 * kg + (r & 3)];
+                    if (dst != kNoStore)
+                        a.y[size_t(dst & 0x7fffffffu) * a.N + col] =
+                            (dst >> 31) ? uint16_t(float_to_half_bits(MEMBER == IQ2_K ? acc[b][mb][r] : acc[b][mb][r] * d))
+                                        : kHalfNaN;
+                }
+            }
+        }
+    };
+    const uint32_t slots = gend - m0;
+    // the empty asm keeps the forms' code apart (merged ahead of the branches
+    // it costs each of them registers)
+    if (slots > 96u) {
+        asm volatile("" ::"n"(4));
+        run(std::integral_constant<int, 4>{});
+    } else if (slots > 64u) {
+        asm volatile("" ::"n"(3));
+        run(std::integral_constant<int, 3>{});
+    } else if (slots > 32u) {
+        asm volatile("" ::"n"(2));
+        run(std::integral_constant<int, 2>{});
+    } else {
+        asm volatile("" ::"n"(1));
+        run(std::integral_constant<int, 1>{});
+    }
+}
+
+// Calls of many slots take the wide tiles: kWideMinSlots a group on average,
+// and kWideMinWork slots x column blocks, three rounds of the 512 blocks the
+// chip holds.  Measured (64-slot tiles -> wide, the kernel alone; routing
+// uniform unless Zipf): IQ2_K gate, 256 experts, Zipf, 192 slots a group 1024
+// -> 940 us, IQ2_KS 954 -> 926; 64 experts, 768: 844 -> 774; 32, 1536: 840 ->
+// 763 (1081 TFLOP/s); IQ2_K down, 160, 230: 776 -> 719; IQ1_S_R4 gate, 128,
+// Zipf, 384: 884 -> 815.  Below the line: 256 experts at 144 (a full wide
+// tile and 16 more) 761 -> 807, at 48 328 -> 380; 32 experts at 192 (0.75 of a
+// round) 143 -> 154.  A launch of their own for the rests measured the same or
+// slower (32 experts, 192: 166; 128, Zipf, 384: 850 us).
+constexpr uint64_t kWideMinSlots = 160;
+constexpr uint64_t kWideMinWork = 3 * 512 * uint64_t(kWideBM);
+
+template <int MEMBER, int K>
+int launch_fused(const FusedArgs &a, hipStream_t st) {
+    const uint64_t ncb = (a.N + kFusedBN - 1) / kFusedBN, slots = a.n_slots, groups = a.n_groups;
+    static_assert(kWideBN == kFusedBN, "both forms cut the rows alike");
+    const bool wide = slots >= kWideMinSlots * groups && slots * ncb >= kWideMinWork;
+    // tiles an XCD: of the 64-slot cut; or of the wide tiles (each of more
+    // than 64 slots) and the rests (at most one a group)
+    const uint64_t share = wide ? (std::min(slots / (kFusedBM + 1), slots / kWideBM + groups) + 7) / 8 +
+                                      (std::min(slots, groups) + 7) / 8
+                                : ((slots + kFusedBM - 1) / kFusedBM + groups + 7) / 8;
+    const uint64_t blocks = 8 * share * ncb;
     if (blocks > 0x7fffffffull) return IQK_ERR_ARGUMENT;
-    const dim3 grid{uint32_t(blocks)}, block{kFusedThreads};
-    if (k == 4096)
-        hipLaunchKernelGGL((fused_gemm_kernel<MEMBER, 4096>), grid, block, 0, st, a);
+    if (wide)
+        hipLaunchKernelGGL((wide_gemm_kernel<MEMBER, K>), dim3{uint32_t(blocks)}, dim3{kWideThreads}, 0, st, a);
     else
-        hipLaunchKernelGGL((fused_gemm_kernel<MEMBER, 2048>), grid, block, 0, st, a);
+        hipLaunchKernelGGL((fused_gemm_kernel<MEMBER, K>), dim3{uint32_t(blocks)}, dim3{kFusedThreads}, 0, st, a);
     return record_launch(hipGetLastError());
 }
 
@@ -1034,9 +1392,10 @@ extern "C" int iqk_fused_gemm(int member, int64_t in_features, int64_t out_featu
     a.n_slots = uint32_t(n_slots);
     a.n_x_rows = uint32_t(n_x_rows);
     hipStream_t st = as_stream(stream);
+    const bool w4096 = in_features == 4096;
     switch (member) {
-        case IQK_MEMBER_IQ2_KS: return launch_fused<IQ2_KS>(in_features, a, uint32_t(n_slots), st);
-        case IQK_MEMBER_IQ2_K: return launch_fused<IQ2_K>(in_features, a, uint32_t(n_slots), st);
-        default: return launch_fused<IQ1_S_R4>(in_features, a, uint32_t(n_slots), st);
+        case IQK_MEMBER_IQ2_KS: return w4096 ? launch_fused<IQ2_KS, 4096>(a, st) : launch_fused<IQ2_KS, 2048>(a, st);
+        case IQK_MEMBER_IQ2_K: return w4096 ? launch_fused<IQ2_K, 4096>(a, st) : launch_fused<IQ2_K, 2048>(a, st);
+        default: return w4096 ? launch_fused<IQ1_S_R4, 4096>(a, st) : launch_fused<IQ1_S_R4, 2048>(a, st);
     }
 }

@@ -2,7 +2,9 @@
 
 A tile holds up to 64 slots of one expert; tiles of at most 8, at most 16, at
 most 32 and more slots run different code, and the work list is scanned in one
-pass for up to 512 experts.  One call here has experts of every count around
+pass for up to 512 experts.  Calls of many slots take 128-slot tiles, whose
+32-slot blocks run different code too, in a list scanned 256 experts a pass.
+One call here has experts of every count around
 those edges, over whole and partial blocks of 256 weight rows, with a slot
 without an activation row; every output is compared with a float64
 contraction of the oracle's weights.
@@ -88,3 +90,64 @@ def test_more_experts_than_one_scan(device, experts):
     module, ref = _module("iq2_ks", experts, 16, 2048, 7, device)
     got, x, xr = _call(module, counts, device, 11, 0, 16, dead=3)
     _check(got, x, xr, counts, ref, dead=3)
+
+
+def _check_on_device(y, x, xr, counts, weights, dead, device):
+    """_check with the float64 contraction on the device, expert by expert."""
+    at = 0
+    for e, c in enumerate(counts):
+        rows = np.arange(at, at + c)
+        at += c
+        rows = rows[rows != dead]
+        if not rows.size:
+            continue
+        w = torch.from_numpy(weights[e]).to(device).double()
+        want = torch.from_numpy(x[xr[rows]]).to(device).double() @ w.T.contiguous()
+        got = y[torch.from_numpy(rows).to(device)].double()
+        assert bool((got - want).abs().max() <= 2e-3 * want.abs().max()), e
+    assert bool(torch.isnan(y[dead]).all())
+
+
+def _wide_call(module, counts, device, seed, row_start, rows, dead):
+    rng = np.random.default_rng(seed)
+    P, n, n_x = int(np.sum(counts)), module.in_features, 509
+    x = rng.standard_normal((n_x, n)).astype(np.float16)
+    xr = rng.integers(0, n_x, P).astype(np.int32)
+    xr[dead] = n_x
+    yr = rng.permutation(P).astype(np.int32)
+    offs = np.concatenate([[0], np.cumsum(counts)]).astype(np.int32)
+    args = [torch.from_numpy(a).to(device) for a in (x, offs, xr, yr)]
+    call = lambda: kernels.fused_matmul(module.member, args[0], module._streams(), module.num_experts,  # noqa: E731
+                                        module.out_features, *args[1:], row_start=row_start, rows=rows)
+    y = call()
+    assert torch.equal(y.view(torch.int16), call().view(torch.int16))
+    return y[args[3].long()], x, xr
+
+
+# around every 32-slot block of a wide tile, and experts of few slots and none
+WIDE_COUNTS = [1280 + c for c in (0, 1, 31, 33, 64, 65, 96, 97, 127)] + [0, 1, 20, 40, 64, 65, 128, 129]
+
+
+@pytest.mark.parametrize("member", fmt.MEMBERS)
+@pytest.mark.parametrize("n", kernels.SUPPORTED_IN_FEATURES)
+@pytest.mark.parametrize("row_start,rows", [(0, 4096), (9, 4080)])
+def test_wide_tiles_match_float64(device, member, n, row_start, rows):
+    """12,481 slots of 17 experts over 16 blocks of weight rows."""
+    print(f"wide tiles {member} n={n} rows [{row_start}, +{rows}]", flush=True)
+    seed = wirepack.seed_for(member, n, "wide")
+    module, ref = _module(member, len(WIDE_COUNTS), 4096, n, seed, device)
+    assert sum(WIDE_COUNTS) >= 160 * len(WIDE_COUNTS) and 16 * sum(WIDE_COUNTS) >= 3 * 512 * 128
+    dead = 1280 + 5
+    y, x, xr = _wide_call(module, WIDE_COUNTS, device, seed, row_start, rows, dead)
+    _check_on_device(y, x, xr, WIDE_COUNTS, ref[:, row_start:row_start + rows], dead, device)
+
+
+def test_wide_tiles_over_more_experts_than_one_scan(device):
+    print("wide tiles over 260 experts", flush=True)
+    rng = np.random.default_rng(3)
+    counts = rng.integers(650, 950, 260)
+    counts[[3, 255, 256, 259]] = [0, 129, 7, 1500]
+    module, ref = _module("iq2_ks", 260, 256, 2048, 5, device)
+    assert counts.sum() >= 3 * 512 * 128
+    y, x, xr = _wide_call(module, counts, device, 13, 0, 256, dead=700)
+    _check_on_device(y, x, xr, counts, ref, 700, device)
