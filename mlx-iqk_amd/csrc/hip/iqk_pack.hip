@@ -6,12 +6,20 @@
 // pack's, bit for bit.
 //
 // A block takes whole wire rows (IQ1_S_R4: whole four-row groups), copies
-// their contiguous wire bytes into LDS with dword loads (a block's rows start
+// their contiguous wire bytes into LDS with 16-byte loads (a block's rows start
 // 4-byte aligned: it takes an even number of rows, and every wire row is an
-// even number of bytes), and then one thread per 256-weight block (IQ1_S_R4:
-// per 32-weight block of a group) reads its bytes from LDS and writes its
-// share of every output plane; consecutive threads write consecutive bytes of
-// each plane's row.
+// even number of bytes), and then one thread per half of a 256-weight block
+// (IQ1_S_R4: per 32-weight block of a group) reads its bytes from LDS and
+// writes its share of every output plane; consecutive threads write consecutive
+// bytes of each plane's row (the two threads of a block exchange half their
+// words, so a code store covers 32 bytes a pair).
+//
+// Bound by the bytes in and out; what stood above that was the relayout's VALU
+// work (each 2-bit field gathered by itself, 450 a block; transposed, 160), a
+// thread's four 16-byte stores 64 bytes apart and dword loads.  64 experts
+// [4096 x 2048], IQ2_K: 81.0 -> 60.6 us (5.26 TB/s read + written; a plain copy
+// runs at 4.6), IQ2_KS 78.2 -> 59.3.  About 256 items a block: 512 took 64.7 us,
+// 1024 69.7; non-temporal stores 74.4.
 //
 // 2-bit members: wire qs byte 32h + 16f + j (h, f in {0,1}, j < 16) carries
 // in field s (bits 2s, 2s+1) the code of weight 128h + 32s + 16f + j, so
@@ -27,7 +35,7 @@ namespace iqk {
 
 constexpr int kPackThreads = 256;
 constexpr int kPackLdsBytes = 40960;
-constexpr int kPackBatch = 8;  // wire dwords a thread loads before it stores them
+constexpr int kPackBatch = 4;  // 16-byte wire pieces a thread loads before it stores them
 
 struct PackArgs {
     const uint8_t *wire;
@@ -50,23 +58,32 @@ __device__ __forceinline__ void lds_words(const uint8_t *lds, uint32_t off, uint
     }
 }
 
-// Field s of the four bytes of q, packed as four 2-bit codes (byte k's field
-// at bits 2k, 2k+1).
-__device__ __forceinline__ uint32_t gather_field(uint32_t q, int s) {
-    const uint32_t t = (q >> (2 * s)) & 0x03030303u;
-    const uint32_t u = t | (t >> 6);
-    return (u | (u >> 12)) & 0xffu;
+// The 4 x 4 transpose of q's 2-bit fields: byte s of the result holds field s
+// of the four bytes of q (byte k's at bits 2k, 2k+1).
+__device__ __forceinline__ uint32_t transpose_fields(uint32_t q) {
+    uint32_t t = (q ^ (q >> 6)) & 0x00CC00CCu;
+    q ^= t ^ (t << 6);
+    t = (q ^ (q >> 12)) & 0x0000F0F0u;
+    return q ^ t ^ (t << 12);
 }
 
-// The 16 relayout words of one 256-weight block from its 64 wire qs bytes.
-__device__ __forceinline__ void relayout_codes(const uint32_t *q, uint32_t *out) {
+// Fields 0 .. 3 of 16 wire bytes as relayout words: 40 VALU for four words
+// (gathering each field of each dword by itself took 112).
+__device__ __forceinline__ void relayout_half(const uint32_t *q, uint32_t *out) {
+    uint32_t t[4];
 #pragma unroll
-    for (int w = 0; w < 16; ++w) {
-        const uint32_t *src = q + 8 * (w >> 3) + 4 * (w & 1);  // wire bytes 32h + 16f .. +15
-        const int s = (w >> 1) & 3;
-        out[w] = gather_field(src[0], s) | (gather_field(src[1], s) << 8) | (gather_field(src[2], s) << 16) |
-                 (gather_field(src[3], s) << 24);
-    }
+    for (int i = 0; i < 4; ++i) t[i] = transpose_fields(q[i]);
+    const uint32_t a = perm(t[1], t[0], 0x05010400u), b = perm(t[3], t[2], 0x05010400u);  // bytes 0, 1
+    const uint32_t c = perm(t[1], t[0], 0x07030602u), d = perm(t[3], t[2], 0x07030602u);  // bytes 2, 3
+    out[0] = perm(b, a, 0x05040100u);
+    out[1] = perm(b, a, 0x07060302u);
+    out[2] = perm(d, c, 0x05040100u);
+    out[3] = perm(d, c, 0x07060302u);
+}
+
+// The value of the other lane of a pair (DPP quad_perm [1,0,3,2]).
+__device__ __forceinline__ uint32_t pair_swap(uint32_t v) {
+    return uint32_t(__builtin_amdgcn_mov_dpp(int(v), 0xB1, 0xF, 0xF, false));
 }
 
 template <int MEMBER>
@@ -80,57 +97,78 @@ __global__ __launch_bounds__(kPackThreads) void pack_kernel(PackArgs a) {
     const uint64_t first = uint64_t(r0) * a.row_bytes;  // 4-byte aligned (even rows per block, even row bytes)
     const uint32_t bytes = rows_here * a.row_bytes;
     const uint32_t *src = reinterpret_cast<const uint32_t *>(a.wire + first);
-    // in batches of kPackBatch loads a thread, all issued before any store,
-    // so the copy costs a memory latency a batch, not one per dword
-    const uint32_t words = bytes / 4;
-    for (uint32_t i0 = 0; i0 < words; i0 += kPackBatch * kPackThreads) {
-        uint32_t v[kPackBatch];
+    // in batches of kPackBatch 16-byte loads a thread (dword aligned), all
+    // issued before any store, so the copy costs a memory latency a batch
+    const uint32_t quads = bytes / 16;
+    for (uint32_t i0 = 0; i0 < quads; i0 += kPackBatch * kPackThreads) {
+        uint4_t v[kPackBatch];
 #pragma unroll
         for (int j = 0; j < kPackBatch; ++j) {
             const uint32_t i = i0 + uint32_t(j * kPackThreads + tid);
-            v[j] = src[min(i, words - 1u)];  // past the end: re-reads the last dword, never stored
+            v[j] = load_u4(src + 4 * min(i, quads - 1u));  // past the end: re-reads the last one, never stored
         }
 #pragma unroll
         for (int j = 0; j < kPackBatch; ++j) {
             const uint32_t i = i0 + uint32_t(j * kPackThreads + tid);
-            if (i < words) reinterpret_cast<uint32_t *>(lds)[i] = v[j];
+            if (i < quads) reinterpret_cast<uint4_t *>(lds)[i] = v[j];
         }
     }
+    if (tid < int(bytes / 4 - 4 * quads)) reinterpret_cast<uint32_t *>(lds)[4 * quads + tid] = src[4 * quads + tid];
     if ((bytes & 3u) && tid == 0)  // an odd last row leaves one 16-bit unit
         *reinterpret_cast<uint16_t *>(lds + (bytes & ~3u)) = *reinterpret_cast<const uint16_t *>(a.wire + first + (bytes & ~3u));
     __syncthreads();
 
     if constexpr (MEMBER == IQ2_KS || MEMBER == IQ2_K) {
-        const uint32_t items = rows_here * a.nb;
+        // an item is half a block: 32 wire qs bytes, 8 relayout words.  Lanes
+        // go in pairs (whole blocks), so every lane of a pair has an item.
+        const uint32_t items = 2 * rows_here * a.nb;
         for (uint32_t it = tid; it < items; it += kPackThreads) {
-            const uint32_t rl = it / a.nb, b = it - rl * a.nb;
+            const uint32_t rl = it / (2 * a.nb), b = (it >> 1) - rl * a.nb, half = it & 1u;
             const uint64_t row = r0 + rl;
             const uint32_t rbase = rl * a.row_bytes;
-            uint32_t q[16], words[16];
+            uint32_t q[8];
             if constexpr (MEMBER == IQ2_KS) {  // [d f16] then blocks [extra u16, scales[4], qs[64]]
                 const uint32_t off = rbase + 2 + 70 * b;
-                uint32_t hdr[2];
-                lds_words(lds, off, hdr, 2);
-                lds_words(lds, off + 6, q, 16);
-                static_cast<uint8_t *>(a.s3)[row * a.nb + b] = uint8_t(hdr[0]);        // sex: extra low byte
-                static_cast<uint8_t *>(a.s2)[row * a.nb + b] = uint8_t(hdr[0] >> 8);   // sch: extra high byte
-                static_cast<uint32_t *>(a.s1)[row * a.nb + b] = __builtin_amdgcn_alignbyte(hdr[1], hdr[0], 2);  // scales[4]
-                if (b == 0) static_cast<uint16_t *>(a.s4)[row] = *reinterpret_cast<const uint16_t *>(lds + rbase);
-            } else {  // blocks [d f16, extra u16, scales[8], qs[64]]
-                const uint32_t off = rbase + 76 * b;
-                uint32_t hdr[3];
-                lds_words(lds, off, hdr, 3);
-                lds_words(lds, off + 12, q, 16);
-                static_cast<uint16_t *>(a.s3)[row * a.nb + b] = uint16_t(hdr[0]);            // dv
-                static_cast<uint16_t *>(a.s2)[row * a.nb + b] = uint16_t(hdr[0] >> 16);      // sex, 2 bytes (LE)
-                uint32_t *scl = reinterpret_cast<uint32_t *>(static_cast<uint8_t *>(a.s1) + (row * a.nb + b) * 8);
-                scl[0] = hdr[1];
-                scl[1] = hdr[2];
-            }
-            relayout_codes(q, words);
-            uint4_t *qs = reinterpret_cast<uint4_t *>(static_cast<uint32_t *>(a.s0) + (row * a.nb + b) * 16);
+                lds_words(lds, off + 6 + 32 * half, q, 8);
+                if (half == 0) {
+                    uint32_t hdr[2];
+                    lds_words(lds, off, hdr, 2);
+                    static_cast<uint8_t *>(a.s3)[row * a.nb + b] = uint8_t(hdr[0]);        // sex: extra low byte
+                    static_cast<uint8_t *>(a.s2)[row * a.nb + b] = uint8_t(hdr[0] >> 8);   // sch: extra high byte
+                    static_cast<uint32_t *>(a.s1)[row * a.nb + b] = __builtin_amdgcn_alignbyte(hdr[1], hdr[0], 2);  // scales[4]
+                    if (b == 0) static_cast<uint16_t *>(a.s4)[row] = *reinterpret_cast<const uint16_t *>(lds + rbase);
+                }
+            } else {  // blocks [d f16, extra u16, scales[8], qs[64]]: dword aligned
+                const uint32_t *blk = reinterpret_cast<const uint32_t *>(lds + rbase + 76 * b);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) qs[i] = uint4_t{words[4 * i], words[4 * i + 1], words[4 * i + 2], words[4 * i + 3]};
+                for (int i = 0; i < 8; ++i) q[i] = blk[3 + 8 * half + i];
+                if (half == 0) {
+                    const uint32_t hdr = blk[0];
+                    static_cast<uint16_t *>(a.s3)[row * a.nb + b] = uint16_t(hdr);            // dv
+                    static_cast<uint16_t *>(a.s2)[row * a.nb + b] = uint16_t(hdr >> 16);      // sex, 2 bytes (LE)
+                    uint32_t *scl = reinterpret_cast<uint32_t *>(static_cast<uint8_t *>(a.s1) + (row * a.nb + b) * 8);
+                    scl[0] = blk[1];
+                    scl[1] = blk[2];
+                }
+            }
+            // words 2s + f of the half: field s of its bytes 16f .. 16f + 15
+            uint32_t w0[4], w1[4];
+            relayout_half(q, w0);
+            relayout_half(q + 4, w1);
+            // The pair's 64 bytes, lane by lane: each store instruction writes
+            // 32 contiguous bytes a pair, the first one the even lane's half.
+            uint32_t keep[4], send[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const uint32_t lo = i & 1 ? w1[i >> 1] : w0[i >> 1];          // words 0 .. 3 of the half
+                const uint32_t hi = i & 1 ? w1[2 + (i >> 1)] : w0[2 + (i >> 1)];  // words 4 .. 7
+                keep[i] = half ? hi : lo;
+                send[i] = pair_swap(half ? lo : hi);
+            }
+            uint4_t *qs = reinterpret_cast<uint4_t *>(static_cast<uint32_t *>(a.s0) + (row * a.nb + b) * 16);
+            const uint4_t own = {keep[0], keep[1], keep[2], keep[3]}, other = {send[0], send[1], send[2], send[3]};
+            qs[half] = half ? other : own;      // even half: words 0 .. 3 | 4 .. 7
+            qs[2 + half] = half ? own : other;  // odd half
         }
     } else {  // IQ1_S_R4: groups [d f16 x4] then blocks [qs[16] (byte 4t + k: row k), qh u16 x4]
         const uint32_t gbytes = 4 * a.row_bytes;
@@ -185,7 +223,7 @@ extern "C" int iqk_pack(int member, int64_t in_features, int64_t rows, const voi
     // rows per block: an even number (a multiple of 4 for IQ1_S_R4) whose bytes fit the LDS copy,
     // about 256 work items per block
     const int64_t unit = iq1 ? 4 : 2;
-    const int64_t per_unit_items = iq1 ? nb : 2 * nb;
+    const int64_t per_unit_items = iq1 ? nb : 4 * nb;
     int64_t units = std::max<int64_t>(1, kPackThreads / per_unit_items);
     units = std::min<int64_t>(units, kPackLdsBytes / (unit * row_bytes));
     if (units < 1) return IQK_ERR_GEOMETRY;  // one row group does not fit the LDS copy
