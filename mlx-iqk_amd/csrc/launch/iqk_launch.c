@@ -1,7 +1,7 @@
-/* A CPython binding of the decode GEMV entry points of libiqk_hip.so: the
- * launch path an eager decode call takes (a 1-token dispatch's kernel runs
- * for ~6 us, and a ctypes call with twelve converted arguments costs ~4 us of
- * host time).  Each function takes the C ABI's arguments as Python integers
+/* A CPython binding of the decode, verify and prefill entry points of
+ * libiqk_hip.so: the launch paths an eager call of the switch module takes (a
+ * 1-token dispatch's kernel runs for ~6 us, and a ctypes call with twelve
+ * converted arguments costs ~4 us of host time).  Each function takes the C ABI's arguments as Python integers
  * (device pointers as addresses, the stream as its handle) and returns the
  * entry point's code; nothing else is done here.  It is built against the
  * library's own header and carries the digest of the sources it was built
@@ -57,6 +57,63 @@ static PyObject *gemv(PyObject *self, PyObject *const *args, Py_ssize_t nargs) {
     return PyLong_FromLong(rc);
 }
 
+static PyObject *refuse(const char *what) {
+    PyErr_SetString(PyExc_OverflowError, what);
+    return NULL;
+}
+
+/* sorted(union, member, n, out, num_experts, x, n_x_rows, streams, n_streams,
+ *        sorted_ids, toks, mats, y, stream): iqk_gemv_sorted, or iqk_gemv_union. */
+static PyObject *sorted(PyObject *self, PyObject *const *args, Py_ssize_t nargs) {
+    (void)self;
+    if (nargs != 14) {
+        PyErr_SetString(PyExc_TypeError, "sorted takes 14 integer arguments");
+        return NULL;
+    }
+    long long v[14];
+    for (int i = 0; i < 14; ++i)
+        if (!as_i64(args[i], &v[i])) return NULL;
+    if (v[1] < INT_MIN || v[1] > INT_MAX || v[8] < INT_MIN || v[8] > INT_MAX || v[11] < 0 || v[11] > UINT32_MAX)
+        return refuse("sorted: member, stream count or pair count out of range");
+    const int rc = (v[0] ? iqk_gemv_union : iqk_gemv_sorted)(
+        (int)v[1], (int64_t)v[2], (int64_t)v[3], (int64_t)v[4], (const void *)(uintptr_t)v[5], (int64_t)v[6],
+        (const void *const *)(uintptr_t)v[7], (int)v[8], (const uint32_t *)(uintptr_t)v[9],
+        (const uint32_t *)(uintptr_t)v[10], (uint32_t)v[11], (void *)(uintptr_t)v[12], (void *)(uintptr_t)v[13]);
+    return PyLong_FromLong(rc);
+}
+
+/* prefill(member, n, out, num_experts, x, n_x_rows, streams, n_streams,
+ *         row_start, rows, ids, wide, n_pairs, rows_per_pair, pairs_per_x_row,
+ *         work, y, stream): iqk_route (wide: iqk_route_ids64), then
+ * iqk_fused_gemm on its lists, which take 2 n_pairs rows_per_pair +
+ * num_experts + 1 words of work.  The first code other than IQK_OK. */
+static PyObject *prefill(PyObject *self, PyObject *const *args, Py_ssize_t nargs) {
+    (void)self;
+    if (nargs != 18) {
+        PyErr_SetString(PyExc_TypeError, "prefill takes 18 integer arguments");
+        return NULL;
+    }
+    long long v[18];
+    for (int i = 0; i < 18; ++i)
+        if (!as_i64(args[i], &v[i])) return NULL;
+    if (v[0] < INT_MIN || v[0] > INT_MAX || v[7] < INT_MIN || v[7] > INT_MAX)
+        return refuse("prefill: member or stream count out of range");
+    /* the lists' addresses need the product; iqk_route refuses the same values */
+    if (v[12] < 0 || v[12] > INT_MAX || v[13] <= 0 || v[13] > INT_MAX) return PyLong_FromLong(IQK_ERR_ARGUMENT);
+    const int64_t slots = (int64_t)v[12] * (int64_t)v[13];
+    uint32_t *x_rows = (uint32_t *)(uintptr_t)v[15], *y_rows = x_rows + slots, *offsets = y_rows + slots;
+    void *stream = (void *)(uintptr_t)v[17];
+    int rc = v[11] ? iqk_route_ids64((const int64_t *)(uintptr_t)v[10], (int64_t)v[12], (int64_t)v[3], (int64_t)v[13],
+                                     (int64_t)v[14], (int64_t)v[5], offsets, x_rows, y_rows, stream)
+                   : iqk_route((const uint32_t *)(uintptr_t)v[10], (int64_t)v[12], (int64_t)v[3], (int64_t)v[13],
+                               (int64_t)v[14], (int64_t)v[5], offsets, x_rows, y_rows, stream);
+    if (rc == IQK_OK)
+        rc = iqk_fused_gemm((int)v[0], (int64_t)v[1], (int64_t)v[2], (int64_t)v[3], (const void *)(uintptr_t)v[4],
+                            (int64_t)v[5], (const void *const *)(uintptr_t)v[6], (int)v[7], (int64_t)v[8],
+                            (int64_t)v[9], offsets, x_rows, y_rows, slots, (void *)(uintptr_t)v[16], stream);
+    return PyLong_FromLong(rc);
+}
+
 static PyObject *source_hash(PyObject *self, PyObject *unused) {
     (void)self;
     (void)unused;
@@ -65,6 +122,8 @@ static PyObject *source_hash(PyObject *self, PyObject *unused) {
 
 static PyMethodDef methods[] = {
     {"gemv", (PyCFunction)(void (*)(void))gemv, METH_FASTCALL, "iqk_gemv / _floor / _floor_grid / _ids64"},
+    {"sorted", (PyCFunction)(void (*)(void))sorted, METH_FASTCALL, "iqk_gemv_sorted / _union"},
+    {"prefill", (PyCFunction)(void (*)(void))prefill, METH_FASTCALL, "iqk_route / _ids64, then iqk_fused_gemm"},
     {"source_hash", source_hash, METH_NOARGS, "digest of the kernel sources this binding was built with"},
     {NULL, NULL, 0, NULL},
 };

@@ -233,8 +233,7 @@ def gemv_checked(member: str, x: torch.Tensor, streams: "CheckedStreams", sel: t
     the reshapes and repeated checks of :func:`gemv`.)"""
     if not mats:
         return
-    stream = (_raw_stream(streams.device_index) if _raw_stream is not None
-              else torch.cuda.current_stream(streams.device).cuda_stream)
+    stream = _current_stream(streams)
     kind = 3 if wide else 0
     fast = _native.launcher()
     if fast is not None and mats <= 65535:  # one launch: the binding's call with nothing else around it
@@ -516,6 +515,52 @@ def route_ids(ids: torch.Tensor, num_experts: int, rows_per_pair: int = 1, pairs
     if rc:
         _native.check(rc, f"iqk_route(P={P}, E={E}, M={M})")
     return offs, x_rows, y_rows
+
+
+def _current_stream(streams: "CheckedStreams") -> int:
+    return (_raw_stream(streams.device_index) if _raw_stream is not None
+            else torch.cuda.current_stream(streams.device).cuda_stream)
+
+
+def gemv_sorted_checked(member: str, x: torch.Tensor, streams: "CheckedStreams", ids: torch.Tensor,
+                        toks: torch.Tensor, x_rows: int, out: torch.Tensor, union: bool) -> bool:
+    """:func:`gemv_sorted` into ``out`` for operands the caller has checked (an
+    IQ2 member, x fp16, ids and toks int32 of one length, all contiguous and on
+    the streams' GPU, ``streams.gemv_ok``); False where the launch binding is
+    not built, with nothing launched."""
+    fast = _native.launcher()
+    if fast is None:
+        return False
+    _, experts, rows, n = streams.key
+    rc = fast.sorted(union, _native.MEMBER_IDS[member], n, rows, experts, x.data_ptr(), x_rows, streams.ptrs_addr,
+                     streams.count, ids.data_ptr(), toks.data_ptr(), out.shape[0], out.data_ptr(),
+                     _current_stream(streams))
+    if rc:
+        _native.check(rc, f"iqk_gemv_{'union' if union else 'sorted'}({member}, {n}x{rows})")
+    return True
+
+
+def prefill_checked(member: str, x: torch.Tensor, streams: "CheckedStreams", ids: torch.Tensor, wide: bool,
+                    n_x_rows: int, n_pairs: int, rows_per_pair: int, pairs_per_x_row: int, row_start: int, rows: int,
+                    out: torch.Tensor) -> bool:
+    """:func:`route_ids` and :func:`fused_matmul` in one call of the launch
+    binding, their lists in one workspace, for operands the caller has checked:
+    x fp16 with ``n_x_rows`` rows, ids int32 (``wide``: int64), out fp16 with
+    ``n_pairs x rows_per_pair x rows`` elements, all contiguous and on the
+    streams' GPU, and :func:`fused_fits`; False where the binding is not built,
+    with nothing launched."""
+    fast = _native.launcher()
+    if fast is None:
+        return False
+    _, experts, out_features, n = streams.key
+    work = torch.empty(2 * n_pairs * rows_per_pair + experts + 1, dtype=torch.int32, device=streams.device)
+    rc = fast.prefill(_native.MEMBER_IDS[member], n, out_features, experts, x.data_ptr(), n_x_rows, streams.ptrs_addr,
+                      streams.count, row_start, rows, ids.data_ptr(), wide, n_pairs, rows_per_pair, pairs_per_x_row,
+                      work.data_ptr(), out.data_ptr(), _current_stream(streams))
+    if rc:
+        _native.check(rc, f"iqk_route / iqk_fused_gemm({member}, {n}x{out_features}, P={n_pairs}, E={experts}, "
+                          f"M={rows_per_pair})")
+    return True
 
 
 FUSED_MEMBERS = MEMBERS

@@ -38,6 +38,21 @@ from .kernels import IqkKernelError, check_dequant_geometry, check_gemv_geometry
 _KERNEL_IDS = {torch.int32: False, torch.int64: True}
 """Id types the decode and the route kernels read as they are: whether wide."""
 
+
+def _pairs_per_x_row(xbatch: tuple, batch: tuple) -> int | None:
+    """The pairs of ``batch`` that one activation row of ``xbatch`` serves,
+    consecutive ones: xbatch equals batch up to some dimension and is 1 (or
+    absent) from there on.  None where it broadcasts otherwise."""
+    absent = len(batch) - len(xbatch)
+    if absent < 0:
+        return None
+    pad = (1,) * absent + tuple(xbatch)
+    lead = 0
+    while lead < len(batch) and pad[lead] == batch[lead]:
+        lead += 1
+    return math.prod(batch[lead:]) if all(d == 1 for d in pad[lead:]) else None
+
+
 DECODE_MAT_LIMIT = 63
 """Token-expert pairs at or below which the decode GEMV serves
 (reference: src/mlx_iqk/nn.py:49-54)."""
@@ -265,9 +280,7 @@ class IqkSwitchLinear(torch.nn.Module):
         result is the pair GEMV's rows in the caller's sorted order.  IQ2
         members only.
         """
-        xt, sel, tok = self._sorted_operands(x, sorted_ids, toks)
-        return kernels.gemv_sorted(self.member, xt, self._checked(), sel, tok, self.num_experts,
-                                   self.out_features)
+        return self._gemv_sorted(x, sorted_ids, toks, False)
 
     def gemv_union(self, x: torch.Tensor, sorted_ids: torch.Tensor, toks: torch.Tensor) -> torch.Tensor:
         """:meth:`gemv_sorted` decoding each run of equal adjacent ids
@@ -276,9 +289,24 @@ class IqkSwitchLinear(torch.nn.Module):
         :meth:`gemv_sorted` bit for bit; three adjacent pairs share a
         workgroup, which loads and expands the rows of each run of one expert
         among them once.  The caller applies the inverse permutation."""
+        return self._gemv_sorted(x, sorted_ids, toks, True)
+
+    def _gemv_sorted(self, x: torch.Tensor, sorted_ids: torch.Tensor, toks: torch.Tensor, union: bool) -> torch.Tensor:
+        chk = self._checked()
+        mats = sorted_ids.numel()
+        # operands in the kernel's layout launch as they are (as in gemv):
+        # 7.4 us of host time a call, 13.6 by the general form
+        if (x.dtype == torch.float16 and sorted_ids.dtype == torch.int32 and toks.dtype == torch.int32
+                and 0 < mats <= 65535 and toks.numel() == mats and chk.gemv_ok and self.member in kernels.IQ2_MEMBERS
+                and x.shape[-1:] == (self.in_features,)
+                and x.is_contiguous() and sorted_ids.is_contiguous() and toks.is_contiguous()
+                and x.get_device() == sorted_ids.get_device() == toks.get_device() == chk.device_index):
+            out = torch.empty((mats, self.out_features), dtype=torch.float16, device=chk.device)
+            if kernels.gemv_sorted_checked(self.member, x, chk, sorted_ids, toks, x.numel() // self.in_features, out,
+                                           union):
+                return out
         xt, sel, tok = self._sorted_operands(x, sorted_ids, toks)
-        return kernels.gemv_sorted(self.member, xt, self._checked(), sel, tok, self.num_experts,
-                                   self.out_features, union=True)
+        return kernels.gemv_sorted(self.member, xt, chk, sel, tok, self.num_experts, self.out_features, union=union)
 
     def _device_ids(self, indices: torch.Tensor) -> torch.Tensor:
         """Expert ids as the kernels read them (32-bit, compared unsigned with
@@ -322,6 +350,9 @@ class IqkSwitchLinear(torch.nn.Module):
     def _sorted_matmul(self, x: torch.Tensor, indices: torch.Tensor, start: int, rows: int) -> torch.Tensor:
         if x.shape[-1] != self.in_features or x.dim() < 2:
             raise IqkRuntimeError(f"x must be [..., M, {self.in_features}], got {tuple(x.shape)}")
+        y = self._fused_as_is(x, indices, start, rows)
+        if y is not None:
+            return y
         device = self.qs.device
         xb = x.to(torch.float16)
         M = int(xb.shape[-2])
@@ -352,6 +383,35 @@ class IqkSwitchLinear(torch.nn.Module):
         y = kernels.grouped_gemm(xflat, w, slot_offsets, x_rows, y_rows)
         return y.reshape(tuple(batch) + (M, rows))
 
+    def _fused_as_is(self, x: torch.Tensor, indices: torch.Tensor, start: int, rows: int) -> torch.Tensor | None:
+        """The fused route for operands already in the kernels' layout: fp16
+        contiguous x, int32 or int64 contiguous ids, on the streams' GPU, x's
+        batch shape equal to the ids' or 1 from some dimension on.  None for
+        any other, with nothing launched.  The general route's reshapes,
+        broadcasts, checks and two ctypes calls took 34 us of host time a
+        call, more than a short prompt's kernels; this takes 13."""
+        wide = _KERNEL_IDS.get(indices.dtype)
+        if not (x.dtype == torch.float16 and wide is not None and self.fused_prefill
+                and self.member in kernels.FUSED_MEMBERS and self.num_experts <= kernels.ROUTE_MAX_EXPERTS
+                and x.is_contiguous() and indices.is_contiguous()):
+            return None
+        if not x.is_cuda:
+            return None
+        chk = self._checked()
+        if not (x.get_device() == indices.get_device() == chk.device_index):
+            return None
+        batch, pairs, n_x_rows = indices.shape, indices.numel(), x.numel() // self.in_features
+        if pairs == 0 or not kernels.fused_fits(n_x_rows, self.in_features, self.out_features):
+            return None
+        M, per_row = x.shape[-2], _pairs_per_x_row(x.shape[:-2], batch)
+        if per_row is None:
+            return None
+        y = torch.empty((*batch, M, rows), dtype=torch.float16, device=chk.device)
+        if not kernels.prefill_checked(self.member, x, chk, indices, wide, n_x_rows, pairs, M, per_row,
+                                       start, rows, y):
+            return None
+        return y
+
     def _route(self, xbatch: tuple, batch: tuple, indices: torch.Tensor, M: int, n_x_rows: int):
         """Group offsets (per expert, in slots) and each slot's activation and
         output row, slots sorted by expert.  An id outside [0, E) reaches no
@@ -364,15 +424,12 @@ class IqkSwitchLinear(torch.nn.Module):
         # pairs per activation row when x broadcasts over trailing batch dims
         # only (gate/up: x [T, 1, 1, in] with indices [T, k]; sorted pairs:
         # x [P, 1, in] with indices [P]): then one device launch does it all
-        pad = (1,) * (len(batch) - len(xbatch)) + tuple(xbatch)
-        lead = 0
-        while lead < len(batch) and pad[lead] == batch[lead]:
-            lead += 1
-        if all(d == 1 for d in pad[lead:]) and E <= kernels.ROUTE_MAX_EXPERTS:
+        per_row = _pairs_per_x_row(xbatch, batch)
+        if per_row is not None and E <= kernels.ROUTE_MAX_EXPERTS:
             ids = indices.to(device).broadcast_to(batch).reshape(-1)
             if ids.dtype not in _KERNEL_IDS or not ids.is_contiguous():
                 ids = self._device_ids(ids)
-            return kernels.route_ids(ids, E, M, math.prod(batch[lead:]), n_x_rows)
+            return kernels.route_ids(ids, E, M, per_row, n_x_rows)
         xidx = torch.arange(math.prod(xbatch), device=device).reshape(xbatch).broadcast_to(batch).reshape(-1)
         raw = indices.to(device=device, dtype=torch.int64).broadcast_to(batch).reshape(-1)
         valid = (raw >= 0) & (raw < E)
