@@ -233,6 +233,17 @@ int iqk_route_ids64(const int64_t *ids, int64_t n_pairs, int64_t num_experts, in
                     int64_t pairs_per_x_row, int64_t n_x_rows, uint32_t *group_offsets, uint32_t *x_rows,
                     uint32_t *y_rows, void *stream);
 
+// The prefill of a switch module in one call: iqk_route (wide_ids: iqk_route_ids64)
+// over n_pairs ids, then iqk_fused_gemm on its lists, with the outputs and
+// refusals of the two.  work: u32 [2 n_pairs rows_per_pair + num_experts + 1]
+// for the lists.  Small calls (at most 1024 pairs of one row, 512 experts and
+// 1536 blocks) take one launch, whose blocks find their own pairs (work is not
+// written).
+int iqk_prefill(int member, int64_t in_features, int64_t out_features, int64_t num_experts, const void *x,
+                int64_t n_x_rows, const void *const *streams, int n_streams, int64_t row_start, int64_t rows,
+                const void *ids, int wide_ids, int64_t n_pairs, int64_t rows_per_pair, int64_t pairs_per_x_row,
+                uint32_t *work, void *y, void *stream);
+
 // ik wire rows -> the member's relayout streams, on the GPU (replaces
 // format.pack for rows already in device memory, src/mlx_iqk/format.py:478-588,
 // 612-678): the bytes pack writes, bit for bit.  wire: u8 [rows, ik row bytes]

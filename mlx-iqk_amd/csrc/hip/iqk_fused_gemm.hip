@@ -47,6 +47,7 @@
 // one 16-code word, with the block's pool of exact products (2s+1)(g +
 // shift), the row's d applied to the sums as for IQ2_KS.
 
+#include <algorithm>
 #include <type_traits>
 
 #include "iqk_device.h"
@@ -85,6 +86,10 @@ struct FusedArgs {
     uint32_t out_rows;  // rows per expert in the streams
     uint32_t row_start;
     uint32_t n_groups, n_slots, n_x_rows;
+    // null, or the pairs' expert ids (64-bit: wide_ids), slot lists and offsets
+    // then unused: each block finds its tile's pairs itself (count_pairs, list_pairs)
+    const uint32_t *ids;
+    uint32_t wide_ids, pairs_per_row;
 };
 
 // How a launch cuts a group's slots into tiles.
@@ -111,12 +116,12 @@ struct FusedScan {
 // The group of an XCD's nth tile, and the tile's number within it: XCD x takes
 // tiles x ceil(T / 8) .. of the list's T, in group order.  False (uniformly)
 // past its share.  Up to a group a thread, the sizes are loaded and scanned
-// once, for T and the tile both.  share: ceil(T / 8).
-template <int CUT, int THREADS>
-__device__ __forceinline__ bool claim_tile(const uint32_t *offs, uint32_t n_groups, uint32_t xcd, uint32_t nth,
+// once, for T and the tile both.  size_of: a group's slots; share: ceil(T / 8).
+template <int CUT, int THREADS, class SizeOf>
+__device__ __forceinline__ bool claim_tile(SizeOf size_of, uint32_t n_groups, uint32_t xcd, uint32_t nth,
                                            FusedScan &ts, uint32_t &group, uint32_t &mtile, uint32_t &share) {
     const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const auto tiles_at = [&](uint32_t g) { return g < n_groups ? tiles_of<CUT>(offs[g + 1] - offs[g]) : 0u; };
+    const auto tiles_at = [&](uint32_t g) { return g < n_groups ? tiles_of<CUT>(size_of(g)) : 0u; };
     const bool once = n_groups <= uint32_t(THREADS);  // uniform
     uint32_t total = 0;
     if (!once) {
@@ -557,9 +562,9 @@ struct FewShape {
     static constexpr int UNITS = 2 * PHASE / 16;     // 16-byte units a row
 };
 
-template <int MEMBER, int K, int ROWS, int PC>
-__device__ __forceinline__ void few_slots_tile(const FusedArgs &a, uint8_t *xs, uint32_t *slot_dst, uint32_t *slot_x,
-                                               const uint2_t *ptab, const uint2_t *grid, uint32_t m0, uint32_t gend,
+template <int MEMBER, int K, int ROWS, int PC, class RowsOf>
+__device__ __forceinline__ void few_slots_tile(const FusedArgs &a, RowsOf rows_of, uint8_t *xs, uint32_t *slot_dst,
+                                               uint32_t *slot_x, const uint2_t *ptab, const uint2_t *grid, uint32_t m0, uint32_t gend,
                                                uint32_t n0, int rows_here, size_t row0, int tid) {
     constexpr bool IQ1 = MEMBER == IQ1_S_R4;
     using F = FewShape<MEMBER, K, ROWS, PC>;
@@ -582,7 +587,8 @@ __device__ __forceinline__ void few_slots_tile(const FusedArgs &a, uint8_t *xs, 
         const uint32_t xp = m0 + uint32_t(tid);
         uint32_t off = xbytes, dst = kNoStore;
         if (xp < gend) {
-            const uint32_t row = a.xr[xp], yrow = a.yr ? a.yr[xp] : xp;
+            uint32_t row, yrow;
+            rows_of(xp, row, yrow);
             if (row < a.n_x_rows) off = row * uint32_t(2 * K);
             if (yrow < a.n_slots) dst = yrow | (row < a.n_x_rows ? 0x80000000u : 0u);  // else NaN
         }
@@ -686,7 +692,67 @@ __device__ __forceinline__ void few_slots_tile(const FusedArgs &a, uint8_t *xs, 
     }
 }
 
-template <int MEMBER, int K>
+// ---- a block's own routing --------------------------------------------------------
+
+// Small calls (takes_own_routing) need no route launch: each block counts the
+// pairs of every expert, finds its tile from the counts, and lists its tile's
+// pairs.  That reads the ids (8 KB at most, from L2) in place of the offsets,
+// and replaces two dependent loads of the slots' rows.
+constexpr uint32_t kSelfPairs = 2 * kFusedThreads, kSelfExperts = kFusedThreads;
+
+// Expert of each of the thread's pairs (0, with bit 31, for an id that names
+// none; 0xffffffff past the last pair), and the experts' pair counts.
+__device__ __forceinline__ void count_pairs(const FusedArgs &a, uint32_t *sizes, uint32_t (&key)[kSelfPairs / kFusedThreads],
+                                            int tid) {
+    sizes[tid] = 0;
+    uint32_t id[kSelfPairs / kFusedThreads];
+#pragma unroll
+    for (uint32_t i = 0; i < kSelfPairs / kFusedThreads; ++i) {
+        const uint32_t p = min(uint32_t(tid) + kFusedThreads * i, a.n_slots - 1u);
+        id[i] = a.ids[p << a.wide_ids];
+        if (a.wide_ids && a.ids[2 * p + 1]) id[i] = 0xffffffffu;
+    }
+    __syncthreads();
+#pragma unroll
+    for (uint32_t i = 0; i < kSelfPairs / kFusedThreads; ++i) {
+        key[i] = id[i] < a.n_groups ? id[i] : 0x80000000u;
+        if (uint32_t(tid) + kFusedThreads * i < a.n_slots)
+            atomicAdd(&sizes[key[i] & 0x7fffffffu], 1u);
+        else
+            key[i] = 0xffffffffu;
+    }
+    __syncthreads();
+}
+
+// Pairs m0 .. m0 + kFusedBM - 1 of group g, in pair order, bit 31 where the id
+// named no expert.  counts: a word a wavefront.
+__device__ __forceinline__ void list_pairs(const FusedArgs &a, const uint32_t (&key)[kSelfPairs / kFusedThreads],
+                                           uint32_t g, uint32_t m0, uint32_t *pairs, uint32_t *counts, int tid) {
+    const int lane = tid & 63, wave = tid >> 6;
+    uint32_t before = 0;  // of the earlier pieces
+#pragma unroll
+    for (uint32_t i = 0; i < kSelfPairs / kFusedThreads; ++i) {
+        if (kFusedThreads * i >= a.n_slots) break;  // uniform
+        const bool mine = key[i] != 0xffffffffu && (key[i] & 0x7fffffffu) == g;
+        const uint64_t m = __ballot(mine);
+        __syncthreads();  // the counts' last readers (the sizes', before the first)
+        if (lane == 0) counts[wave] = uint32_t(__popcll(m));
+        __syncthreads();
+        uint32_t at = before;
+#pragma unroll
+        for (int w = 0; w < kFusedWaves; ++w) {
+            if (w < wave) at += counts[w];
+            before += counts[w];
+        }
+        at += __builtin_amdgcn_mbcnt_hi(uint32_t(m >> 32), __builtin_amdgcn_mbcnt_lo(uint32_t(m), 0u)) - m0;
+        if (mine && at < uint32_t(kFusedBM)) pairs[at] = (uint32_t(tid) + kFusedThreads * i) | (key[i] & 0x80000000u);
+    }
+    __syncthreads();
+}
+
+// SELF: each block finds its tile's pairs from a.ids (a kernel of its own, so
+// the listed form's code is unchanged).
+template <int MEMBER, int K, bool SELF>
 __global__ __launch_bounds__(kFusedThreads) __attribute__((amdgpu_waves_per_eu(4)))
 void fused_gemm_kernel(FusedArgs a) {
     constexpr bool IQ1 = MEMBER == IQ1_S_R4;
@@ -704,6 +770,7 @@ void fused_gemm_kernel(FusedArgs a) {
     // are real (else its output row is NaN), or kNoStore
     __shared__ uint32_t slot_dst[kFusedBM];
     __shared__ uint32_t slot_x[kFewSlots];
+    __shared__ uint32_t pairs[SELF ? kFusedBM : 1];
     __shared__ uint2_t ptab[MEMBER == IQ2_K ? 32 : IQ1 ? 16 : 64];  // pool products (IQ2_K) or pools
     // Phases of a few-slot tile: 64 KB of activations beside the tables leave
     // two blocks a CU; IQ1_S_R4's grid leaves room for 32 KB.
@@ -724,8 +791,12 @@ void fused_gemm_kernel(FusedArgs a) {
     const int tid = threadIdx.x;
     const uint32_t ncb = (a.N + kFusedBN - 1) / kFusedBN;  // column blocks
     const uint32_t xcd = blockIdx.x & 7u, j = blockIdx.x >> 3, cblock = j % ncb;
+    uint32_t *const sizes = reinterpret_cast<uint32_t *>(fxs);  // SELF: every group's, until the tile's pairs are listed
+    uint32_t key[kSelfPairs / kFusedThreads];                   // SELF: of pairs tid + 512 i
+    if constexpr (SELF) count_pairs(a, sizes, key, tid);
+    const auto size_of = [&](uint32_t e) { return SELF ? sizes[e] : a.offs[e + 1] - a.offs[e]; };
     uint32_t g, mtile, share;
-    if (!claim_tile<kCut64, kFusedThreads>(a.offs, a.n_groups, xcd, j / ncb, ts, g, mtile, share)) return;  // surplus
+    if (!claim_tile<kCut64, kFusedThreads>(size_of, a.n_groups, xcd, j / ncb, ts, g, mtile, share)) return;  // surplus
 
     // Offsets and row indices are device data: a slot outside [0, n_slots)
     // is never stored, a row outside x is never read (its output row is NaN),
@@ -733,8 +804,21 @@ void fused_gemm_kernel(FusedArgs a) {
     // rows read an in-bounds row instead, so the step has no branches but
     // (IQ1_S_R4) the one that skips staging activation rows past the tile's
     // end.
-    const uint32_t gend = min(a.offs[g + 1], a.n_slots);
-    const uint32_t m0 = a.offs[g] + mtile * kFusedBM;
+    // (SELF: slots count from the group's first)
+    const uint32_t gend = SELF ? __builtin_amdgcn_readfirstlane(sizes[g]) : min(a.offs[g + 1], a.n_slots);
+    const uint32_t m0 = (SELF ? 0u : a.offs[g]) + mtile * kFusedBM;
+    if constexpr (SELF) list_pairs(a, key, g, m0, pairs, ts.wave, tid);
+    // slot xp's activation row (none: past x) and output row
+    const auto rows_of = [&](uint32_t xp, uint32_t &row, uint32_t &yrow) {
+        if constexpr (SELF) {
+            const uint32_t p = pairs[xp - m0];
+            yrow = p & 0x7fffffffu;
+            row = (p >> 31) ? a.n_x_rows : yrow / a.pairs_per_row;
+        } else {
+            row = a.xr[xp];
+            yrow = a.yr ? a.yr[xp] : xp;
+        }
+    };
     const uint32_t n0 = cblock * kFusedBN;
     const int rows_here = int(min(uint32_t(kFusedBN), a.N - n0));
     const size_t row0 = size_t(g) * a.out_rows + a.row_start + n0;  // first stacked weight row of the block
@@ -757,12 +841,12 @@ void fused_gemm_kernel(FusedArgs a) {
     // apart: merged ahead of the branches it costs each of them registers.
     if (gend - m0 <= 8u) {
         asm volatile("" ::"n"(8));
-        few_slots_tile<MEMBER, K, 8, PC8>(a, fxs, slot_dst, slot_x, ptab, grid, m0, gend, n0, rows_here, row0, tid);
+        few_slots_tile<MEMBER, K, 8, PC8>(a, rows_of, fxs, slot_dst, slot_x, ptab, grid, m0, gend, n0, rows_here, row0, tid);
         return;
     }
     if (gend - m0 <= uint32_t(kFewSlots)) {
         asm volatile("" ::"n"(16));
-        few_slots_tile<MEMBER, K, 16, P8 / 2>(a, fxs, slot_dst, slot_x, ptab, grid, m0, gend, n0, rows_here, row0, tid);
+        few_slots_tile<MEMBER, K, 16, P8 / 2>(a, rows_of, fxs, slot_dst, slot_x, ptab, grid, m0, gend, n0, rows_here, row0, tid);
         return;
     }
     // scale planes of the block's rows
@@ -797,7 +881,8 @@ void fused_gemm_kernel(FusedArgs a) {
     for (int i = 0; i < kXPer; ++i) {
         const int row = xrow_l + kXRows * i;
         const uint32_t xp = m0 + uint32_t(row);
-        const uint32_t xrow = xp < gend ? a.xr[xp] : a.n_x_rows;
+        uint32_t xrow = a.n_x_rows, yrow = kNoStore;
+        if (xp < gend) rows_of(xp, xrow, yrow);
         const bool xv = xrow < a.n_x_rows;
         // a dead slot reads row 0 (the entry point refuses an empty x); its
         // products feed only its own output row, never stored as a value
@@ -806,12 +891,7 @@ void fused_gemm_kernel(FusedArgs a) {
         xoff[i] = (xv ? xrow : 0u) * uint32_t(2 * K) + uint32_t(16 * xchunk) + (xchunk >= 8 ? 128u * (G - 1) : 0u);
         xlive[i] = !IQ1 || xp < gend;
         if (xchunk == 0) {  // one thread a slot: the epilogue's destination, read once
-            uint32_t dst = kNoStore;
-            if (xp < gend) {
-                const uint32_t yrow = a.yr ? a.yr[xp] : xp;
-                if (yrow < a.n_slots) dst = yrow | (xv ? 0x80000000u : 0u);
-            }
-            slot_dst[row] = dst;
+            slot_dst[row] = yrow < a.n_slots ? yrow | (xv ? 0x80000000u : 0u) : kNoStore;
         }
     }
     // Staging pass i covers slot block i (rows 32i .. 32i+31): a tile of
@@ -1111,12 +1191,13 @@ void wide_gemm_kernel(FusedArgs a) {
     const uint32_t ncb = (a.N + kWideBN - 1) / kWideBN;
     // the wide tiles first (the long ones), then the rests
     const uint32_t xcd = blockIdx.x & 7u, nth = (blockIdx.x >> 3) / ncb, cblock = (blockIdx.x >> 3) % ncb;
+    const auto size_of = [&](uint32_t e) { return a.offs[e + 1] - a.offs[e]; };
     uint32_t g, mtile, share;
-    if (!claim_tile<kCutWide, kWideThreads>(a.offs, a.n_groups, xcd, nth, ts, g, mtile, share)) {
+    if (!claim_tile<kCutWide, kWideThreads>(size_of, a.n_groups, xcd, nth, ts, g, mtile, share)) {
         if (nth < share) return;  // uniform
         __syncthreads();          // the first claim's totals have been read
         const uint32_t wide = share;
-        if (!claim_tile<kCutRest, kWideThreads>(a.offs, a.n_groups, xcd, nth - wide, ts, g, mtile, share)) return;
+        if (!claim_tile<kCutRest, kWideThreads>(size_of, a.n_groups, xcd, nth - wide, ts, g, mtile, share)) return;
         mtile = (a.offs[g + 1] - a.offs[g]) / kWideBM;
     }
     const uint32_t gend = min(a.offs[g + 1], a.n_slots);
@@ -1337,33 +1418,59 @@ void wide_gemm_kernel(FusedArgs a) {
 constexpr uint64_t kWideMinSlots = 160;
 constexpr uint64_t kWideMinWork = 3 * 512 * uint64_t(kWideBM);
 
+inline bool takes_wide_tiles(uint64_t rows, uint64_t slots, uint64_t groups) {
+    static_assert(kWideBN == kFusedBN, "both forms cut the rows alike");
+    const uint64_t ncb = (rows + kFusedBN - 1) / kFusedBN;
+    return slots >= kWideMinSlots * groups && slots * ncb >= kWideMinWork;
+}
+
+// An upper bound on the 64-slot tiles of a call.
+inline uint64_t most_tiles(uint64_t slots, uint64_t groups) {
+    return std::min(slots, (slots + kFusedBM - 1) / kFusedBM + groups);
+}
+
+// Calls whose blocks route for themselves (count_pairs, list_pairs): one
+// block's routing takes about 1 us where the launch it replaces took 3 to 4, so
+// it pays for about three rounds of the 512 blocks the chip holds.  Measured
+// (route launch -> own, us a call): 32 experts, 4 of 24 to 149 tokens, up to
+// 736 blocks, IQ2_KS gate 29.5 -> 26.9, 33.6 -> 30.6, 36.1 -> 33.5, IQ1_S_R4
+// down 27.1 -> 23.6, 28.9 -> 25.2, 34.4 -> 31.6; 256 experts, 6 of 12 and 24
+// tokens, Zipf, 576 and 1152 blocks, gate: 44.0 -> 41.2, 49.2 -> 46.2.  Past the
+// line: 96 experts, down, 1664 blocks: 68.8 -> 72.7; 256 experts, down, 4192
+// blocks: IQ1_S_R4 127.9 -> 135.1.
+constexpr uint64_t kSelfBlocks = 3 * 512;
+
+inline bool takes_own_routing(uint64_t rows, uint64_t slots, uint64_t groups) {
+    const uint64_t ncb = (rows + kFusedBN - 1) / kFusedBN;
+    return slots <= kSelfPairs && groups <= kSelfExperts && most_tiles(slots, groups) * ncb <= kSelfBlocks &&
+           !takes_wide_tiles(rows, slots, groups);
+}
+
 template <int MEMBER, int K>
 int launch_fused(const FusedArgs &a, hipStream_t st) {
     const uint64_t ncb = (a.N + kFusedBN - 1) / kFusedBN, slots = a.n_slots, groups = a.n_groups;
-    static_assert(kWideBN == kFusedBN, "both forms cut the rows alike");
-    const bool wide = slots >= kWideMinSlots * groups && slots * ncb >= kWideMinWork;
+    const bool wide = takes_wide_tiles(a.N, slots, groups);
     // tiles an XCD: of the 64-slot cut; or of the wide tiles (each of more
     // than 64 slots) and the rests (at most one a group)
     const uint64_t share = wide ? (std::min(slots / (kFusedBM + 1), slots / kWideBM + groups) + 7) / 8 +
                                       (std::min(slots, groups) + 7) / 8
-                                : ((slots + kFusedBM - 1) / kFusedBM + groups + 7) / 8;
+                                : (most_tiles(slots, groups) + 7) / 8;
     const uint64_t blocks = 8 * share * ncb;
     if (blocks > 0x7fffffffull) return IQK_ERR_ARGUMENT;
     if (wide)
         hipLaunchKernelGGL((wide_gemm_kernel<MEMBER, K>), dim3{uint32_t(blocks)}, dim3{kWideThreads}, 0, st, a);
+    else if (a.ids)
+        hipLaunchKernelGGL((fused_gemm_kernel<MEMBER, K, true>), dim3{uint32_t(blocks)}, dim3{kFusedThreads}, 0, st, a);
     else
-        hipLaunchKernelGGL((fused_gemm_kernel<MEMBER, K>), dim3{uint32_t(blocks)}, dim3{kFusedThreads}, 0, st, a);
+        hipLaunchKernelGGL((fused_gemm_kernel<MEMBER, K, false>), dim3{uint32_t(blocks)}, dim3{kFusedThreads}, 0, st, a);
     return record_launch(hipGetLastError());
 }
 
-}  // namespace iqk
-
-extern "C" int iqk_fused_gemm(int member, int64_t in_features, int64_t out_features, int64_t num_experts,
-                              const void *x, int64_t n_x_rows, const void *const *streams, int n_streams,
-                              int64_t row_start, int64_t rows, const uint32_t *group_offsets,
-                              const uint32_t *x_rows, const uint32_t *y_rows, int64_t n_slots, void *y,
-                              void *stream) {
-    using namespace iqk;
+// Slot lists and offsets, or (ids set) the pairs' ids.
+int fused_entry(int member, int64_t in_features, int64_t out_features, int64_t num_experts,
+                const void *x, int64_t n_x_rows, const void *const *streams, int n_streams, int64_t row_start,
+                int64_t rows, const uint32_t *group_offsets, const uint32_t *x_rows, const uint32_t *y_rows,
+                int64_t n_slots, void *y, void *stream, const void *ids, bool wide_ids, int64_t pairs_per_row) {
     if (!member_ok(member)) return IQK_ERR_MEMBER;
     if (!width_sized(in_features)) return IQK_ERR_GEOMETRY;
     if (out_features <= 0 || out_features > (int64_t(1) << 24)) return IQK_ERR_GEOMETRY;
@@ -1374,7 +1481,7 @@ extern "C" int iqk_fused_gemm(int member, int64_t in_features, int64_t out_featu
     if (n_slots < 0 || n_slots > (int64_t(1) << 30) || n_x_rows < 0 || n_x_rows > 0xffffffffll)
         return IQK_ERR_ARGUMENT;
     if (n_slots == 0) return IQK_OK;
-    if (!x || !y || !group_offsets || !x_rows || !streams_ok(streams, n_streams, member)) return IQK_ERR_ARGUMENT;
+    if (!x || !y || (!ids && (!group_offsets || !x_rows)) || !streams_ok(streams, n_streams, member)) return IQK_ERR_ARGUMENT;
     if (n_x_rows == 0 || n_x_rows * in_features * 2 >= (int64_t(1) << 32)) return IQK_ERR_ARGUMENT;
     FusedArgs a;
     a.x = static_cast<const uint16_t *>(x);
@@ -1391,6 +1498,9 @@ extern "C" int iqk_fused_gemm(int member, int64_t in_features, int64_t out_featu
     a.n_groups = uint32_t(num_experts);
     a.n_slots = uint32_t(n_slots);
     a.n_x_rows = uint32_t(n_x_rows);
+    a.ids = static_cast<const uint32_t *>(ids);
+    a.wide_ids = wide_ids ? 1u : 0u;
+    a.pairs_per_row = uint32_t(pairs_per_row);
     hipStream_t st = as_stream(stream);
     const bool w4096 = in_features == 4096;
     switch (member) {
@@ -1399,3 +1509,46 @@ extern "C" int iqk_fused_gemm(int member, int64_t in_features, int64_t out_featu
         default: return w4096 ? launch_fused<IQ1_S_R4, 4096>(a, st) : launch_fused<IQ1_S_R4, 2048>(a, st);
     }
 }
+
+}  // namespace iqk
+
+extern "C" {
+
+int iqk_fused_gemm(int member, int64_t in_features, int64_t out_features, int64_t num_experts, const void *x,
+                   int64_t n_x_rows, const void *const *streams, int n_streams, int64_t row_start, int64_t rows,
+                   const uint32_t *group_offsets, const uint32_t *x_rows, const uint32_t *y_rows, int64_t n_slots,
+                   void *y, void *stream) {
+    return iqk::fused_entry(member, in_features, out_features, num_experts, x, n_x_rows, streams, n_streams, row_start,
+                            rows, group_offsets, x_rows, y_rows, n_slots, y, stream, nullptr, false, 1);
+}
+
+int iqk_prefill(int member, int64_t in_features, int64_t out_features, int64_t num_experts, const void *x,
+                int64_t n_x_rows, const void *const *streams, int n_streams, int64_t row_start, int64_t rows,
+                const void *ids, int wide_ids, int64_t n_pairs, int64_t rows_per_pair, int64_t pairs_per_x_row,
+                uint32_t *work, void *y, void *stream) {
+    using namespace iqk;
+    constexpr int64_t kLim = int64_t(1) << 31;
+    // what the route refuses, before a product of its factors or an address of its lists is formed
+    if (n_pairs < 0 || n_pairs >= kLim || rows_per_pair <= 0 || rows_per_pair >= kLim || pairs_per_x_row <= 0 ||
+        pairs_per_x_row >= kLim || n_x_rows < 0 || n_x_rows >= kLim || n_pairs * rows_per_pair >= kLim)
+        return IQK_ERR_ARGUMENT;
+    if (n_pairs == 0) return IQK_OK;
+    if (!ids || !work) return IQK_ERR_ARGUMENT;
+    // every activation row a pair names lies in x
+    if (((n_pairs - 1) / pairs_per_x_row + 1) * rows_per_pair > n_x_rows) return IQK_ERR_ARGUMENT;
+    const int64_t slots = n_pairs * rows_per_pair;
+    if (rows > 0 && num_experts > 0 && rows_per_pair == 1 &&
+        takes_own_routing(uint64_t(rows), uint64_t(slots), uint64_t(num_experts)))
+        return fused_entry(member, in_features, out_features, num_experts, x, n_x_rows, streams, n_streams, row_start,
+                           rows, nullptr, nullptr, nullptr, slots, y, stream, ids, wide_ids != 0, pairs_per_x_row);
+    uint32_t *const x_rows = work, *const y_rows = work + slots, *const offsets = work + 2 * slots;
+    const int rc = wide_ids ? iqk_route_ids64(static_cast<const int64_t *>(ids), n_pairs, num_experts, rows_per_pair,
+                                              pairs_per_x_row, n_x_rows, offsets, x_rows, y_rows, stream)
+                            : iqk_route(static_cast<const uint32_t *>(ids), n_pairs, num_experts, rows_per_pair,
+                                        pairs_per_x_row, n_x_rows, offsets, x_rows, y_rows, stream);
+    if (rc != IQK_OK) return rc;
+    return fused_entry(member, in_features, out_features, num_experts, x, n_x_rows, streams, n_streams, row_start, rows,
+                       offsets, x_rows, y_rows, slots, y, stream, nullptr, false, 1);
+}
+
+}  // extern "C"

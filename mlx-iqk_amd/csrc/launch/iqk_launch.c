@@ -84,9 +84,7 @@ static PyObject *sorted(PyObject *self, PyObject *const *args, Py_ssize_t nargs)
 
 /* prefill(member, n, out, num_experts, x, n_x_rows, streams, n_streams,
  *         row_start, rows, ids, wide, n_pairs, rows_per_pair, pairs_per_x_row,
- *         work, y, stream): iqk_route (wide: iqk_route_ids64), then
- * iqk_fused_gemm on its lists, which take 2 n_pairs rows_per_pair +
- * num_experts + 1 words of work.  The first code other than IQK_OK. */
+ *         work, y, stream): iqk_prefill. */
 static PyObject *prefill(PyObject *self, PyObject *const *args, Py_ssize_t nargs) {
     (void)self;
     if (nargs != 18) {
@@ -98,19 +96,11 @@ static PyObject *prefill(PyObject *self, PyObject *const *args, Py_ssize_t nargs
         if (!as_i64(args[i], &v[i])) return NULL;
     if (v[0] < INT_MIN || v[0] > INT_MAX || v[7] < INT_MIN || v[7] > INT_MAX)
         return refuse("prefill: member or stream count out of range");
-    /* the lists' addresses need the product; iqk_route refuses the same values */
-    if (v[12] < 0 || v[12] > INT_MAX || v[13] <= 0 || v[13] > INT_MAX) return PyLong_FromLong(IQK_ERR_ARGUMENT);
-    const int64_t slots = (int64_t)v[12] * (int64_t)v[13];
-    uint32_t *x_rows = (uint32_t *)(uintptr_t)v[15], *y_rows = x_rows + slots, *offsets = y_rows + slots;
-    void *stream = (void *)(uintptr_t)v[17];
-    int rc = v[11] ? iqk_route_ids64((const int64_t *)(uintptr_t)v[10], (int64_t)v[12], (int64_t)v[3], (int64_t)v[13],
-                                     (int64_t)v[14], (int64_t)v[5], offsets, x_rows, y_rows, stream)
-                   : iqk_route((const uint32_t *)(uintptr_t)v[10], (int64_t)v[12], (int64_t)v[3], (int64_t)v[13],
-                               (int64_t)v[14], (int64_t)v[5], offsets, x_rows, y_rows, stream);
-    if (rc == IQK_OK)
-        rc = iqk_fused_gemm((int)v[0], (int64_t)v[1], (int64_t)v[2], (int64_t)v[3], (const void *)(uintptr_t)v[4],
-                            (int64_t)v[5], (const void *const *)(uintptr_t)v[6], (int)v[7], (int64_t)v[8],
-                            (int64_t)v[9], offsets, x_rows, y_rows, slots, (void *)(uintptr_t)v[16], stream);
+    const int rc = iqk_prefill((int)v[0], (int64_t)v[1], (int64_t)v[2], (int64_t)v[3], (const void *)(uintptr_t)v[4],
+                               (int64_t)v[5], (const void *const *)(uintptr_t)v[6], (int)v[7], (int64_t)v[8],
+                               (int64_t)v[9], (const void *)(uintptr_t)v[10], v[11] != 0, (int64_t)v[12],
+                               (int64_t)v[13], (int64_t)v[14], (uint32_t *)(uintptr_t)v[15],
+                               (void *)(uintptr_t)v[16], (void *)(uintptr_t)v[17]);
     return PyLong_FromLong(rc);
 }
 
@@ -123,7 +113,7 @@ static PyObject *source_hash(PyObject *self, PyObject *unused) {
 static PyMethodDef methods[] = {
     {"gemv", (PyCFunction)(void (*)(void))gemv, METH_FASTCALL, "iqk_gemv / _floor / _floor_grid / _ids64"},
     {"sorted", (PyCFunction)(void (*)(void))sorted, METH_FASTCALL, "iqk_gemv_sorted / _union"},
-    {"prefill", (PyCFunction)(void (*)(void))prefill, METH_FASTCALL, "iqk_route / _ids64, then iqk_fused_gemm"},
+    {"prefill", (PyCFunction)(void (*)(void))prefill, METH_FASTCALL, "iqk_prefill"},
     {"source_hash", source_hash, METH_NOARGS, "digest of the kernel sources this binding was built with"},
     {NULL, NULL, 0, NULL},
 };

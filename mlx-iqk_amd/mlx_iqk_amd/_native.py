@@ -60,6 +60,9 @@ SIGNATURES = {
     "iqk_pack": (c_int, [c_int, c_int64, c_int64, c_void_p, ctypes.POINTER(c_void_p), c_int, c_void_p]),
     "iqk_fused_gemm": (c_int, [c_int, c_int64, c_int64, c_int64, c_void_p, c_int64, ctypes.POINTER(c_void_p),
                                c_int, c_int64, c_int64, c_void_p, c_void_p, c_void_p, c_int64, c_void_p, c_void_p]),
+    "iqk_prefill": (c_int, [c_int, c_int64, c_int64, c_int64, c_void_p, c_int64, ctypes.POINTER(c_void_p), c_int,
+                            c_int64, c_int64, c_void_p, c_int, c_int64, c_int64, c_int64, c_void_p, c_void_p,
+                            c_void_p]),
 }
 
 

@@ -156,3 +156,26 @@ def test_prefill_direct_replays_in_a_graph(device):
         graph.replay()
         assert _same(y, module(x, ids))
         torch.cuda.synchronize()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("member,n", [("iq2_ks", 4096), ("iq2_k", 4096), ("iq2_k", 2048), ("iq1_s_r4", 2048)])
+@pytest.mark.parametrize("pairs,experts", [(1, 1), (63, 512), (64, 3), (511, 2), (512, 256), (513, 9), (1023, 512),
+                                           (1024, 5), (1024, 513), (1025, 5)])
+@pytest.mark.parametrize("wide", (False, True))
+def test_blocks_find_the_pairs_the_route_lists(device, monkeypatch, member, n, pairs, experts, wide):
+    """Around the limits of the one-launch form (1024 pairs, 512 experts): the
+    outputs of the routed form, with ids that name no expert."""
+    print(f"own routing {member} n={n} pairs={pairs} experts={experts} wide={wide}", flush=True)
+    module = _module(member, experts, 48, n, device)
+    rng = np.random.default_rng(pairs + experts)
+    ids = np.minimum(rng.geometric(0.02 if experts > 100 else 0.3, pairs) - 1, experts - 1)  # some experts with many
+    bad = (experts, -1) + (((1 << 32) + 1, -(1 << 63)) if wide else (2**31 - 1, -(2**31)))
+    for at, b in zip(rng.choice(pairs, min(len(bad), pairs // 2), replace=False), bad):
+        ids[at] = b
+    sel = torch.from_numpy(ids).to(device, torch.int64 if wide else torch.int32)
+    x = torch.from_numpy(rng.standard_normal((pairs, 1, n)).astype(np.float16)).to(device)
+    got = module.prefill(x, sel)
+    monkeypatch.setattr(kernels, "prefill_checked", lambda *a: False)
+    assert _same(got, module.prefill(x, sel))
+    assert torch.equal(torch.isnan(got).all(-1).reshape(-1), (sel < 0) | (sel >= experts))
