@@ -881,7 +881,11 @@ enum GemvMode : int {
 // small to give every CU the same number of 32-row workgroups, such as one
 // token's gate alone: 384 of them on 256 CUs).  With T = 1 each thread
 // stages two activation units (N = 4096) and expands twice the grid entries.
-template <int MEMBER, int N, int FLOOR, int MODE, int R, int T = 2>
+// WIDE: 64-bit ids (pairs mode), a kernel of its own: chosen by an argument
+// inside one kernel they cost the 32-bit calls 0.05 us each (a layer's graph of
+// three 23.75 -> 23.91 us; as a kernel of their own 24.1, 24.4 at the same clock
+// without 64-bit ids at all).
+template <int MEMBER, int N, int FLOOR, int MODE, int R, int T = 2, bool WIDE = false>
 __global__ __launch_bounds__((64 * T * Gemv2Shape<MEMBER, N>::KS))
 __attribute__((amdgpu_waves_per_eu(R == 2 ? 5 : 6)))
 void gemv_mfma_kernel(Gemv2Args a) {
@@ -943,7 +947,7 @@ void gemv_mfma_kernel(Gemv2Args a) {
     // An id beyond the stack reads expert 0 (in bounds) and writes NaN rows.
     // No early exit: a branch here would let the compiler sink the loads
     // above behind the wait for the id.
-    const uint32_t e_raw = MODE == kPairs ? expert_id(a.sel, m0, a.wide_ids) : a.sel[m0];
+    const uint32_t e_raw = WIDE ? expert_id(a.sel, m0, 1u) : a.sel[m0];
     const bool valid = e_raw < a.num_experts;  // uniform per workgroup
     const uint32_t e = valid ? e_raw : 0u;
     LaneOf<MEMBER, N> lane[R];  // rows rowg + 16 (R tile + r) + n
@@ -1026,7 +1030,7 @@ void gemv_mfma_kernel(Gemv2Args a) {
 // turn, so the staging's VALU work (a quarter of a single pair's) is shared
 // P ways.  That pays in dispatches of many tokens, where back-to-back
 // workgroups are bound by VALU issue rather than by HBM.
-template <int MEMBER, int N, int FLOOR, int P>
+template <int MEMBER, int N, int FLOOR, int P, bool WIDE = false>
 __global__ __launch_bounds__((Gemv2Shape<MEMBER, N>::THREADS))
 __attribute__((amdgpu_waves_per_eu(6)))
 void gemv_mfma_pairs_kernel(Gemv2Args a) {
@@ -1066,7 +1070,7 @@ void gemv_mfma_pairs_kernel(Gemv2Args a) {
     bool valid[P];  // uniform per workgroup
 #pragma unroll
     for (int p = 0; p < P; ++p) {
-        const uint32_t e_raw = expert_id(a.sel, m0 + p, a.wide_ids);
+        const uint32_t e_raw = WIDE ? expert_id(a.sel, m0 + p, 1u) : a.sel[m0 + p];
         valid[p] = e_raw < a.num_experts;
         e[p] = valid[p] ? e_raw : 0u;
     }
@@ -1277,15 +1281,27 @@ int launch_gemv_mfma(int64_t n, const Gemv2Args &a, uint32_t mats, hipStream_t s
     const dim3 block4096{uint32_t(64 * T * Gemv2Shape<MEMBER, 4096>::KS)},
         block2048{uint32_t(64 * T * Gemv2Shape<MEMBER, 2048>::KS)};
     static_assert(P == 1 || (MODE == kPairs && R == 1 && T == 2), "several pairs a workgroup: pairs mode, one row block");
-    if constexpr (P > 1) {
-        if (n == 4096)
-            hipLaunchKernelGGL((gemv_mfma_pairs_kernel<MEMBER, 4096, FLOOR, P>), grid, block4096, 0, st, a);
+    const auto launch = [&](auto wide) {
+        constexpr bool WIDE = decltype(wide)::value;
+        if constexpr (P > 1) {
+            if (n == 4096)
+                hipLaunchKernelGGL((gemv_mfma_pairs_kernel<MEMBER, 4096, FLOOR, P, WIDE>), grid, block4096, 0, st, a);
+            else
+                hipLaunchKernelGGL((gemv_mfma_pairs_kernel<MEMBER, 2048, FLOOR, P, WIDE>), grid, block2048, 0, st, a);
+        } else if (n == 4096) {
+            hipLaunchKernelGGL((gemv_mfma_kernel<MEMBER, 4096, FLOOR, MODE, R, T, WIDE>), grid, block4096, 0, st, a);
+        } else {
+            hipLaunchKernelGGL((gemv_mfma_kernel<MEMBER, 2048, FLOOR, MODE, R, T, WIDE>), grid, block2048, 0, st, a);
+        }
+    };
+    if constexpr (MODE == kPairs && FLOOR == kDecode) {
+        if (a.wide_ids)
+            launch(std::true_type{});
         else
-            hipLaunchKernelGGL((gemv_mfma_pairs_kernel<MEMBER, 2048, FLOOR, P>), grid, block2048, 0, st, a);
-    } else if (n == 4096) {
-        hipLaunchKernelGGL((gemv_mfma_kernel<MEMBER, 4096, FLOOR, MODE, R, T>), grid, block4096, 0, st, a);
+            launch(std::false_type{});
     } else {
-        hipLaunchKernelGGL((gemv_mfma_kernel<MEMBER, 2048, FLOOR, MODE, R, T>), grid, block2048, 0, st, a);
+        if (a.wide_ids) return IQK_ERR_ARGUMENT;  // only the decode's pairs mode reads 64-bit ids
+        launch(std::false_type{});
     }
     return record_launch(hipGetLastError());
 }
