@@ -198,9 +198,12 @@ int iqk_grouped_gemm(int64_t in_features, int64_t out_features, int64_t n_groups
 // for bit.  IQ2_KS, IQ1_S_R4 (one scale d a row): the sum runs over the
 // exact products n = W / d and is multiplied by d once, so W enters
 // unrounded (a one-hot x row yields iqk_dequant's fp16 weight).  The
-// summation order differs from iqk_dequant + iqk_grouped_gemm; it does not
-// depend on row_start, so row ranges concatenate to the full call bit for
-// bit.  y: f16 [n_slots, rows];
+// summation order differs from iqk_dequant + iqk_grouped_gemm.  It does not
+// depend on row_start or rows, so row ranges concatenate to the full call bit
+// for bit; it does depend on how many slots the call gives the expert (tiles
+// of at most 16 slots sum in an order of their own), so a slot's outputs may
+// differ in their last bits between calls that hold different slots beside it.
+// Calls with the same slots repeat bit for bit.  y: f16 [n_slots, rows];
 // group_offsets: u32 [num_experts + 1] (device, non-decreasing, last =
 // n_slots); x, x_rows, y_rows as iqk_grouped_gemm.  IQK_ERR_GEOMETRY unless
 // 0 <= row_start < row_start + rows <= out_features.  All three members.

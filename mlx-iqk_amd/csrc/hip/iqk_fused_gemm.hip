@@ -90,6 +90,9 @@ struct FusedArgs {
     // then unused: each block finds its tile's pairs itself (count_pairs, list_pairs)
     const uint32_t *ids;
     uint32_t wide_ids, pairs_per_row;
+    // the expert's full rows would take the wide tiles: no tile takes the
+    // few-slot form, whose sums run in another order (see takes_wide_tiles)
+    uint32_t wide_order;
 };
 
 // How a launch cuts a group's slots into tiles.
@@ -839,12 +842,13 @@ void fused_gemm_kernel(FusedArgs a) {
     }
     // Few slots (uniform per block).  The empty asm keeps the forms' code
     // apart: merged ahead of the branches it costs each of them registers.
-    if (gend - m0 <= 8u) {
+    const uint32_t few = a.wide_order ? 0xffffffffu : gend - m0;
+    if (few <= 8u) {
         asm volatile("" ::"n"(8));
         few_slots_tile<MEMBER, K, 8, PC8>(a, rows_of, fxs, slot_dst, slot_x, ptab, grid, m0, gend, n0, rows_here, row0, tid);
         return;
     }
-    if (gend - m0 <= uint32_t(kFewSlots)) {
+    if (few <= uint32_t(kFewSlots)) {
         asm volatile("" ::"n"(16));
         few_slots_tile<MEMBER, K, 16, P8 / 2>(a, rows_of, fxs, slot_dst, slot_x, ptab, grid, m0, gend, n0, rows_here, row0, tid);
         return;
@@ -1103,20 +1107,23 @@ constexpr int kWideThreads = 256;
 constexpr int kWideBN = 256;  // weight rows per block: 64 a wavefront
 
 // One lane's weights of one row (ln) in steps of 128, as the 64-slot tile
-// takes them: lane group kg the sub-blocks 2kg, 2kg + 1 of a step (IQ1_S_R4, whose
-// steps go in pairs: elements 256p + 128kg + 64j .. +63 of pair p in its step
-// j).  Code words a step ahead; scales of four steps at once (the IQ2 members).
+// takes them, so that both sum an element in one order: lane group kg the
+// sub-blocks 2kg, 2kg + 1 of a step (IQ1_S_R4, whose steps go in groups of
+// four: elements 512p + 256kg + 64j .. +63 of group p in its step j).  Code
+// words a step (IQ1_S_R4: two) ahead; scales of four steps at once (the IQ2
+// members).
 template <int MEMBER, int K>
 struct WideLane {
     static constexpr bool IQ1 = MEMBER == IQ1_S_R4, KS = MEMBER == IQ2_KS;
-    uint4_t q;   // IQ2: a step's code words; IQ1_S_R4: a pair's index words
-    uint2_t h;   // IQ1_S_R4: a pair's qh words
+    uint4_t q;   // IQ2: a step's code words; IQ1_S_R4: two steps' index words
+    uint2_t h;   // IQ1_S_R4: two steps' qh words
 
     __device__ __forceinline__ void load(const FewPlanes<MEMBER, K> &pl, uint32_t row, int kg, int s) {
         using P = FewPlanes<MEMBER, K>;
         if constexpr (IQ1) {
-            q = buffer_u4(pl.p[0], row * P::ROW[0] + 16 * kg, 32 * (s >> 1));
-            h = __builtin_amdgcn_raw_buffer_load_b64(pl.p[1], row * P::ROW[1] + 8 * kg, 16 * (s >> 1), 0);
+            const uint32_t p = uint32_t(s) >> 2, t = (uint32_t(s) >> 1) & 1u;  // steps 4p + 2t, 4p + 2t + 1
+            q = buffer_u4(pl.p[0], row * P::ROW[0] + 32 * kg, 64 * p + 16 * t);
+            h = __builtin_amdgcn_raw_buffer_load_b64(pl.p[1], row * P::ROW[1] + 16 * kg, 32 * p + 8 * t, 0);
         } else {
             q = buffer_u4(pl.p[0], row * P::ROW[0] + 16 * kg, 32 * s);
         }
@@ -1237,7 +1244,7 @@ void wide_gemm_kernel(FusedArgs a) {
         const bool live = xp < gend;
         const uint32_t row = live ? a.xr[xp] : a.n_x_rows;
         const bool xv = row < a.n_x_rows;  // else its output is NaN
-        xoff[i] = xv ? row * uint32_t(2 * K) + uint32_t(16 * xchunk) + (IQ1 && xchunk >= 8 ? 128u : 0u) : xbytes;
+        xoff[i] = xv ? row * uint32_t(2 * K) + uint32_t(16 * xchunk) + (IQ1 && xchunk >= 8 ? 384u : 0u) : xbytes;
         if (xchunk == 0) {
             uint32_t dst = kNoStore;
             if (live) {
@@ -1249,7 +1256,7 @@ void wide_gemm_kernel(FusedArgs a) {
     }
     constexpr int BATCH = PASSES / 2;  // rows go in two batches of 64
     const auto load_x = [&](int s, int b, uint4_t (&v)[BATCH]) {
-        const uint32_t off = IQ1 ? uint32_t(512 * (s >> 1) + 128 * (s & 1)) : uint32_t(256 * s);
+        const uint32_t off = IQ1 ? uint32_t(1024 * (s >> 2) + 128 * (s & 3)) : uint32_t(256 * s);
 #pragma unroll
         for (int i = 0; i < BATCH; ++i) v[i] = buffer_u4(xbuf, xoff[BATCH * b + i], off);
     };
@@ -1302,7 +1309,7 @@ void wide_gemm_kernel(FusedArgs a) {
                 if constexpr (IQ1) {
                     const uint32_t hw = i & 1 ? now[b].h.y : now[b].h.x;
 #pragma unroll
-                    for (int t = 0; t < 2; ++t) {  // blocks 2j, 2j + 1 of the pair
+                    for (int t = 0; t < 2; ++t) {  // blocks 2j, 2j + 1 of the two steps
                         const uint32_t qw = now[b].q[2 * (i & 1) + t], h = (hw >> (16 * t)) & 0xffffu;
                         const uint2_t v = ptab[(h >> 12) & 15u];
                         pool[b][2 * t] = {v.x, v.y};
@@ -1354,7 +1361,7 @@ void wide_gemm_kernel(FusedArgs a) {
         };
 #pragma unroll 1
         for (int p = 0; p < STEPS / 4; ++p) {
-            if constexpr (IQ1) {  // a pair's words serve two steps
+            if constexpr (IQ1) {  // a lane's words serve two steps
                 step(p, 0, cur, nxt);
                 step(p, 1, cur, nxt);
                 step(p, 2, nxt, cur);
@@ -1418,6 +1425,15 @@ void wide_gemm_kernel(FusedArgs a) {
 constexpr uint64_t kWideMinSlots = 160;
 constexpr uint64_t kWideMinWork = 3 * 512 * uint64_t(kWideBM);
 
+//
+// The wide tiles and the 64-slot form sum an element in one order, the
+// few-slot form in another.  So a row range below the line, of an expert whose
+// full rows lie above it, keeps to the 64-slot form (wide_order), and ranges
+// concatenate to the full call bit for bit.  That costs a range nothing that
+// shows (8192 tokens Zipf over 256 experts, IQ2_KS gate, 256 rows: 150.3 ->
+// 151.3 us); wide tiles for every range of such an expert would do it too, but
+// a range of few blocks then waits on its longest tile (32 experts, 2048
+// tokens, down, 256 rows: 31 -> 56 us; the first one, 150 -> 166).
 inline bool takes_wide_tiles(uint64_t rows, uint64_t slots, uint64_t groups) {
     static_assert(kWideBN == kFusedBN, "both forms cut the rows alike");
     const uint64_t ncb = (rows + kFusedBN - 1) / kFusedBN;
@@ -1447,9 +1463,10 @@ inline bool takes_own_routing(uint64_t rows, uint64_t slots, uint64_t groups) {
 }
 
 template <int MEMBER, int K>
-int launch_fused(const FusedArgs &a, hipStream_t st) {
+int launch_fused(FusedArgs a, hipStream_t st) {
     const uint64_t ncb = (a.N + kFusedBN - 1) / kFusedBN, slots = a.n_slots, groups = a.n_groups;
     const bool wide = takes_wide_tiles(a.N, slots, groups);
+    a.wide_order = takes_wide_tiles(a.out_rows, slots, groups) ? 1u : 0u;
     // tiles an XCD: of the 64-slot cut; or of the wide tiles (each of more
     // than 64 slots) and the rests (at most one a group)
     const uint64_t share = wide ? (std::min(slots / (kFusedBM + 1), slots / kWideBM + groups) + 7) / 8 +
