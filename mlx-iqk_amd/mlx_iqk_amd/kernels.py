@@ -233,7 +233,8 @@ def gemv_checked(member: str, x: torch.Tensor, streams: "CheckedStreams", sel: t
     the reshapes and repeated checks of :func:`gemv`.)"""
     if not mats:
         return
-    stream = _current_stream(streams)
+    stream = (_raw_stream(streams.device_index) if _raw_stream is not None
+              else torch.cuda.current_stream(streams.device).cuda_stream)
     kind = 3 if wide else 0
     fast = _native.launcher()
     if fast is not None and mats <= 65535:  # one launch: the binding's call with nothing else around it

@@ -248,8 +248,9 @@ class IqkSwitchLinear(torch.nn.Module):
         # int64 contiguous ids, on the streams' GPU) launch without a reshape and
         # with the output allocated in its final shape: the eager decode's
         # host time is mostly such tensor operations.
-        wide = _KERNEL_IDS.get(indices.dtype)
-        if (x.dtype == torch.float16 and wide is not None and chk.gemv_ok
+        ids = indices.dtype
+        wide = ids is torch.int64
+        if (x.dtype is torch.float16 and (wide or ids is torch.int32) and chk.gemv_ok
                 and x.is_contiguous() and indices.is_contiguous() and x.shape[-1] == self.in_features
                 and x.get_device() == chk.device_index and indices.get_device() == chk.device_index):
             mats, rows = indices.numel(), x.numel() // self.in_features
