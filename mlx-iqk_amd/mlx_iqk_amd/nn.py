@@ -293,21 +293,22 @@ class IqkSwitchLinear(torch.nn.Module):
         return self._gemv_sorted(x, sorted_ids, toks, True)
 
     def _gemv_sorted(self, x: torch.Tensor, sorted_ids: torch.Tensor, toks: torch.Tensor, union: bool) -> torch.Tensor:
-        chk = self._checked()
         mats = sorted_ids.numel()
         # operands in the kernel's layout launch as they are (as in gemv):
         # 7.4 us of host time a call, 13.6 by the general form
-        if (x.dtype == torch.float16 and sorted_ids.dtype == torch.int32 and toks.dtype == torch.int32
-                and 0 < mats <= 65535 and toks.numel() == mats and chk.gemv_ok and self.member in kernels.IQ2_MEMBERS
+        if (x.is_cuda and x.dtype == torch.float16 and sorted_ids.dtype == torch.int32 and toks.dtype == torch.int32
+                and 0 < mats <= 65535 and toks.numel() == mats and self.member in kernels.IQ2_MEMBERS
                 and x.shape[-1:] == (self.in_features,)
-                and x.is_contiguous() and sorted_ids.is_contiguous() and toks.is_contiguous()
-                and x.get_device() == sorted_ids.get_device() == toks.get_device() == chk.device_index):
-            out = torch.empty((mats, self.out_features), dtype=torch.float16, device=chk.device)
-            if kernels.gemv_sorted_checked(self.member, x, chk, sorted_ids, toks, x.numel() // self.in_features, out,
-                                           union):
-                return out
+                and x.is_contiguous() and sorted_ids.is_contiguous() and toks.is_contiguous()):
+            chk = self._checked()
+            if chk.gemv_ok and x.get_device() == sorted_ids.get_device() == toks.get_device() == chk.device_index:
+                out = torch.empty((mats, self.out_features), dtype=torch.float16, device=chk.device)
+                if kernels.gemv_sorted_checked(self.member, x, chk, sorted_ids, toks, x.numel() // self.in_features,
+                                               out, union):
+                    return out
         xt, sel, tok = self._sorted_operands(x, sorted_ids, toks)
-        return kernels.gemv_sorted(self.member, xt, chk, sel, tok, self.num_experts, self.out_features, union=union)
+        return kernels.gemv_sorted(self.member, xt, self._checked(), sel, tok, self.num_experts, self.out_features,
+                                   union=union)
 
     def _device_ids(self, indices: torch.Tensor) -> torch.Tensor:
         """Expert ids as the kernels read them (32-bit, compared unsigned with

@@ -71,6 +71,21 @@ def test_pairs_per_x_row_is_the_broadcast():
             assert not any((row == np.arange(row.size) // n).all() for n in range(1, row.size + 1))
 
 
+@pytest.mark.parametrize("member", fmt.MEMBERS)
+@pytest.mark.parametrize("form", ("gemv_sorted", "gemv_union"))
+def test_sorted_forms_name_a_wrong_operand_before_the_device(member, form):
+    """A module in host memory refuses operands that disagree as one on a GPU
+    does, and only then its own streams."""
+    module = IqkSwitchLinear(member, 4, 32, 2048)
+    call, x, ids = getattr(module, form), torch.zeros((2, 2048), dtype=torch.float16), torch.zeros(4, dtype=torch.int32)
+    with pytest.raises(nn.IqkRuntimeError, match="toks carries 3 rows for 4 pairs"):
+        call(x, ids, ids[:3])
+    with pytest.raises(RuntimeError, match="is invalid for input of size"):
+        call(x[:, :100], ids, ids)
+    with pytest.raises(kernels.IqkKernelError, match="must live on a GPU"):
+        call(x, ids, ids)
+
+
 def _module(member, experts, out, n, device):
     wire = wirepack.random_wire(member, experts * out, n, seed=out, scales="serving")
     module = IqkSwitchLinear(member, experts, out, n, device=device)
