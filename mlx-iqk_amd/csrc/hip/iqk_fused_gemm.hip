@@ -536,6 +536,15 @@ struct FewLane {
     __device__ __forceinline__ uint32_t word(int s, int w) const { return q[MEMBER == IQ1_S_R4 ? 0 : s][w]; }
 };
 
+// LDS shape of a few-slot tile: ROWS staged rows, PC chunks of 512 elements a phase.
+template <int ROWS, int PC>
+struct FewShape {
+    static constexpr int PHASE = 512 * PC;           // reduction elements staged at once
+    static constexpr int STRIDE = 2 * PHASE + 16;    // LDS bytes per staged row
+    static constexpr int BYTES = ROWS * STRIDE;
+    static constexpr int UNITS = 2 * PHASE / 16;     // 16-byte units a row
+};
+
 // A tile of at most ROWS (8 or 16) slots against the block's 256 weight rows,
 // on v_mfma_f32_16x16x32_f16.  Most experts of a batch or a short prompt have
 // such tiles only, and the work is then one expansion of every routed weight
@@ -547,9 +556,10 @@ struct FewLane {
 // chunks, as many as 64 KB hold (IQ1_S_R4, beside its grid: 32 KB): between
 // two phases the wavefronts run free of one another.
 //
-// What bounds it: VALU issue.  Taking the loads out leaves 88% of the time,
-// the MFMAs 86%, and 16-row wavefronts at six or eight a SIMD measured the
-// same, as did loads of whole rows turned through LDS.  The line at 16 slots:
+// What bounds it: VALU issue more than anything else, 61 to 65% of a SIMD's
+// time (MFMA 15 to 19).  Taking the loads out leaves 88% of the time, the MFMAs
+// 86%, and 16-row wavefronts at six or eight a SIMD measured the same, as did
+// loads of whole rows turned through LDS.  The line at 16 slots:
 // two 16-slot blocks an operand measured 5% slower than one 32-slot MFMA
 // (1024 tokens, uniform: 24 slots an expert).  Measured (the kernel alone, 256
 // experts, top-6, uniform routing, IQ2_KS gate): 24 tokens 102 -> 84 us, 64
@@ -557,20 +567,12 @@ struct FewLane {
 // 64 tokens 112 -> 94, 512 243 -> 227, IQ1_S_R4 gate 143 -> 123 and 235 -> 205
 // (128 and 512), IQ2_K down 166 -> 157 and 271 -> 254; 2048 tokens 386 -> 369,
 // 377 -> 356, 430 -> 418.
-template <int MEMBER, int K, int ROWS, int PC>
-struct FewShape {
-    static constexpr int PHASE = 512 * PC;           // reduction elements staged at once
-    static constexpr int STRIDE = 2 * PHASE + 16;    // LDS bytes per staged row
-    static constexpr int BYTES = ROWS * STRIDE;
-    static constexpr int UNITS = 2 * PHASE / 16;     // 16-byte units a row
-};
-
 template <int MEMBER, int K, int ROWS, int PC, class RowsOf>
 __device__ __forceinline__ void few_slots_tile(const FusedArgs &a, RowsOf rows_of, uint8_t *xs, uint32_t *slot_dst,
                                                uint32_t *slot_x, const uint2_t *ptab, const uint2_t *grid, uint32_t m0, uint32_t gend,
                                                uint32_t n0, int rows_here, size_t row0, int tid) {
     constexpr bool IQ1 = MEMBER == IQ1_S_R4;
-    using F = FewShape<MEMBER, K, ROWS, PC>;
+    using F = FewShape<ROWS, PC>;
     constexpr int CHUNKS = K / 512;
     static_assert(CHUNKS % 2 == 0 && CHUNKS % PC == 0, "chunks go in pairs, whole phases");
     const int wave = tid >> 6, l = tid & 63, n = l & 15, g = l >> 4;
@@ -778,8 +780,8 @@ void fused_gemm_kernel(FusedArgs a) {
     // Phases of a few-slot tile: 64 KB of activations beside the tables leave
     // two blocks a CU; IQ1_S_R4's grid leaves room for 32 KB.
     constexpr int P8 = IQ1 ? 4 : 8, PC8 = P8 < K / 512 ? P8 : K / 512;
-    using F8 = FewShape<MEMBER, K, 8, PC8>;
-    using F16 = FewShape<MEMBER, K, 16, P8 / 2>;
+    using F8 = FewShape<8, PC8>;
+    using F16 = FewShape<16, P8 / 2>;
     constexpr int GRID_BYTES = IQ1 ? int(sizeof(FusedGrid)) : 0;
     constexpr int XS_BYTES = 2 * kFusedBM * kXStride;
     constexpr int WIDE_BYTES = XS_BYTES + (IQ1 ? 0 : int(sizeof(S)));
@@ -1114,7 +1116,7 @@ constexpr int kWideBN = 256;  // weight rows per block: 64 a wavefront
 // members).
 template <int MEMBER, int K>
 struct WideLane {
-    static constexpr bool IQ1 = MEMBER == IQ1_S_R4, KS = MEMBER == IQ2_KS;
+    static constexpr bool IQ1 = MEMBER == IQ1_S_R4;
     uint4_t q;   // IQ2: a step's code words; IQ1_S_R4: two steps' index words
     uint2_t h;   // IQ1_S_R4: two steps' qh words
 

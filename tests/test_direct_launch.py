@@ -194,3 +194,48 @@ def test_blocks_find_the_pairs_the_route_lists(device, monkeypatch, member, n, p
     monkeypatch.setattr(kernels, "prefill_checked", lambda *a: False)
     assert _same(got, module.prefill(x, sel))
     assert torch.equal(torch.isnan(got).all(-1).reshape(-1), (sel < 0) | (sel >= experts))
+
+
+def _pool_module(member, experts, out, n, device):
+    """Every four rows drawn from 512 random ones."""
+    pool = torch.from_numpy(wirepack.random_wire(member, 512, n, seed=out, scales="serving")).to(device)
+    g = torch.Generator(device=device).manual_seed(experts)
+    pick = torch.randint(128, (experts * out // 4,), generator=g, device=device)
+    module = IqkSwitchLinear(member, experts, out, n, device=device)
+    module.load_wire(pool.view(128, -1)[pick].view(experts * out, -1))
+    return module
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("member", fmt.MEMBERS)
+@pytest.mark.parametrize("out,tokens,top_k,experts,own", [
+    (272, 86, 6, 40, True), (272, 170, 6, 300, True),  # two column blocks, the second of 16 rows; two pieces of pairs
+    (2048, 32, 6, 200, True), (2048, 193, 1, 200, False),  # 192 and 193 tiles of eight column blocks: by pairs
+    (2048, 170, 6, 176, True), (2048, 170, 6, 177, False),  # by experts, pairs sharing activation rows
+])
+@pytest.mark.parametrize("wide", (False, True))
+def test_own_routing_over_column_blocks(device, monkeypatch, member, out, tokens, top_k, experts, own, wide):
+    """The one-launch form over several column blocks and pairs that share an
+    activation row, on both sides of its 1536 blocks: the routed form's
+    outputs, its workspace written by the routed form alone."""
+    print(f"own routing {member} out={out} {tokens}x{top_k} of {experts} wide={wide}", flush=True)
+    pairs, n = tokens * top_k, 2048
+    assert own == (min(pairs, -(-pairs // 64) + experts) * -(-out // 256) <= 1536)
+    module = _pool_module(member, experts, out, n, device)
+    g = torch.Generator(device=device).manual_seed(pairs)
+    x = torch.randn((tokens, 1, 1, n), generator=g, device=device).to(torch.float16)
+    ids = torch.randint(0, experts, (tokens, top_k), generator=g, device=device)
+    ids[::3, 0] = 1  # an expert of many pairs
+    ids[tokens // 2, -1] = experts
+    sel = ids.to(torch.int64 if wide else torch.int32)
+    got = module.prefill(x, sel)
+    chk, work = module._checked(), torch.full((2 * pairs + experts + 1,), -7, dtype=torch.int32, device=device)
+    y = torch.empty_like(got)
+    rc = _native.launcher().prefill(_native.MEMBER_IDS[member], n, out, experts, x.data_ptr(), tokens, chk.ptrs_addr,
+                                    chk.count, 0, out, sel.data_ptr(), wide, pairs, 1, top_k, work.data_ptr(),
+                                    y.data_ptr(), torch.cuda.current_stream().cuda_stream)
+    assert rc == 0 and _same(y, got)
+    assert bool((work == -7).all()) == own
+    monkeypatch.setattr(kernels, "prefill_checked", lambda *a: False)
+    assert _same(got, module.prefill(x, sel))
+    assert torch.equal(torch.isnan(got).all(-1).squeeze(-1), sel == experts)
