@@ -843,7 +843,8 @@ void fused_gemm_kernel(FusedArgs a) {
             grid[4 * tid + i] = grid_selectors(((i < 2 ? cw.x : cw.y) >> (16 * (i & 1))) & 0xffffu);
     }
     // Few slots (uniform per block).  The empty asm keeps the forms' code
-    // apart: merged ahead of the branches it costs each of them registers.
+    // apart: merged ahead of the branches it costs each of them registers
+    // (IQ1_S_R4, at 128 VGPRs, spills one or two even so).
     const uint32_t few = a.wide_order ? 0xffffffffu : gend - m0;
     if (few <= 8u) {
         asm volatile("" ::"n"(8));
@@ -1181,9 +1182,10 @@ struct WideScales {
 // (64 rows at a time, half a step ahead) are the only thing staged.  Groups
 // are cut into 128-slot tiles, a last one of more than 64 slots among them;
 // what is left (at most 64 slots a group) goes last in the list, so the short
-// tiles fill the end of the launch.  It reaches 0.9 to 1.08 PFLOP/s where an
+// tiles fill the end of the launch.  Over the real slots of the calls listed
+// at takes_wide_tiles it reaches 0.86 (many rests) to 1.08 PFLOP/s, where an
 // 8192-wide fp16 library product reaches 1.08 on this card (the clock its
-// power allows).
+// power allows).  IQ2_KS's form holds 256 VGPRs and spills two; the others none.
 template <int MEMBER, int K>
 __global__ __launch_bounds__(kWideThreads) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void wide_gemm_kernel(FusedArgs a) {

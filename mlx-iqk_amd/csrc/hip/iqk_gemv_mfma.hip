@@ -881,10 +881,8 @@ enum GemvMode : int {
 // small to give every CU the same number of 32-row workgroups, such as one
 // token's gate alone: 384 of them on 256 CUs).  With T = 1 each thread
 // stages two activation units (N = 4096) and expands twice the grid entries.
-// WIDE: 64-bit ids (pairs mode), a kernel of its own: chosen by an argument
-// inside one kernel they cost the 32-bit calls 0.05 us each (a layer's graph of
-// three 23.75 -> 23.91 us; as a kernel of their own 24.1, 24.4 at the same clock
-// without 64-bit ids at all).
+// WIDE: 64-bit ids (pairs mode), a kernel of its own, so that the 32-bit ids'
+// kernels stay instruction for instruction what they are without it.
 template <int MEMBER, int N, int FLOOR, int MODE, int R, int T = 2, bool WIDE = false>
 __global__ __launch_bounds__((64 * T * Gemv2Shape<MEMBER, N>::KS))
 __attribute__((amdgpu_waves_per_eu(R == 2 ? 5 : 6)))

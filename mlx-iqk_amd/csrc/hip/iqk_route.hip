@@ -26,10 +26,12 @@
 // Every block runs over the whole id list, and with many pairs its VALU and
 // SALU work on them bounds the time: with a lane's pairs 64 apart, a ballot
 // pair per 64 of them (24 instructions) and the rank from each, 49152 pairs
-// over 256 experts took 18.1 us and over 32 experts 25.1; now 10.7 and
-// 12.2.  Up to 2048 pairs it is latency: four wavefronts of one piece each
-// take 2.9 us at 144 pairs, launch included (eight wavefronts of 32 ballot
-// steps whatever their share: 5.0).
+// over 256 experts took 18.8 us, over 32 experts 24.8 and 12288 over 256 took
+// 7.4; now 11.5, 12.2 and 5.9, and with 64-bit ids, whose list is twice as
+// long, 15.2, 16.1 and 6.8.  Up to 2048 pairs it is latency: four wavefronts of
+// one piece each take 3.2 us at 144 pairs with either ids (eight wavefronts of
+// 32 ballot steps whatever their share: 5.5).  (Medians of 30 dispatches in a
+// kernel trace, 32-bit ids where not said.)
 
 #include "iqk_device.h"
 #include "iqk_host.h"

@@ -226,8 +226,8 @@ def gemv_checked(member: str, x: torch.Tensor, streams: "CheckedStreams", sel: t
     """The decode GEMV into ``out`` for operands the caller has checked: x
     fp16 and contiguous with ``rows`` rows of the streams' width, sel int32
     (``wide``: int64, which the kernel reads itself: without the three
-    launches that clamped and narrowed the ids an eager call takes 8.4 us, not
-    23.5) and contiguous with ``mats`` ids, out fp16 with ``mats x out_features``
+    launches that clamped and narrowed the ids an eager call takes 8.2 us, not
+    23.3) and contiguous with ``mats`` ids, out fp16 with ``mats x out_features``
     elements, all on the streams' GPU, ``streams.gemv_ok`` and
     ``mats % rows == 0``.  (The switch module's eager decode path: it skips
     the reshapes and repeated checks of :func:`gemv`.)"""

@@ -295,7 +295,7 @@ class IqkSwitchLinear(torch.nn.Module):
     def _gemv_sorted(self, x: torch.Tensor, sorted_ids: torch.Tensor, toks: torch.Tensor, union: bool) -> torch.Tensor:
         mats = sorted_ids.numel()
         # operands in the kernel's layout launch as they are (as in gemv):
-        # 7.4 us of host time a call, 13.6 by the general form
+        # 7.8 us of host time a call, 14.0 by the general form
         if (x.is_cuda and x.dtype == torch.float16 and sorted_ids.dtype == torch.int32 and toks.dtype == torch.int32
                 and 0 < mats <= 65535 and toks.numel() == mats and self.member in kernels.IQ2_MEMBERS
                 and x.shape[-1:] == (self.in_features,)
@@ -390,8 +390,9 @@ class IqkSwitchLinear(torch.nn.Module):
         contiguous x, int32 or int64 contiguous ids, on the streams' GPU, x's
         batch shape equal to the ids' or 1 from some dimension on.  None for
         any other, with nothing launched.  The general route's reshapes,
-        broadcasts, checks and two ctypes calls took 34 us of host time a
-        call, more than a short prompt's kernels; this takes 13."""
+        broadcasts, checks and two ctypes calls took 36 us of host time a
+        call (48 with int64 ids), more than a short prompt's kernels; this
+        takes 14, 11 where the blocks route for themselves."""
         wide = _KERNEL_IDS.get(indices.dtype)
         if not (x.dtype == torch.float16 and wide is not None and self.fused_prefill
                 and self.member in kernels.FUSED_MEMBERS and self.num_experts <= kernels.ROUTE_MAX_EXPERTS
